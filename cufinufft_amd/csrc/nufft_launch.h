@@ -20,6 +20,31 @@ constexpr int kErrNoAlloc = 13;  // no-allocation entry: input beyond what is al
 // kernels' static job slot.
 constexpr size_t kMaxLdsBytes = 160 * 1024 - 64;
 
+// Window kernels (win_device.cuh): S[d] first taps per window, nw[d] windows
+// per axis, nkeys in all; the order of the points by window is cut into ranges
+// of equal work, one per wave.  ranges = 0: the plan's points take the
+// per-point kernels.
+struct WinGeom {
+    int S[3] = {1, 1, 1};
+    int nw[3] = {1, 1, 1};
+    int nkeys = 0;
+    int ns = 2;
+    int ranges = 0;
+};
+// The points in window order, as the kernels read them.
+struct WinPts {
+    const void *x;        // T [dim][stride]: first tap - position + ns/2
+    const unsigned *sh;   // first tap inside its window, a byte per axis
+    const int *idx;       // the caller's index
+    const int *start;     // first point of each window (nkeys + 1)
+    const int *range;     // first point of each range (ranges + 1)
+    long long stride;
+};
+constexpr int kWinKeyWeight = 8;  // a window's own time in a range, in points
+// Half of a 3D interp window's y and z extent: windows of 8 cells up to ns 8,
+// of ns + 1 or ns + 2 beyond.
+constexpr int win_interp_half(int ns) { return ns <= 8 ? 4 : (ns + 2) / 2; }
+
 // Device arrays written by setpts.
 struct SortBufs {
     int *binsize = nullptr;     // [nbins]
@@ -41,6 +66,16 @@ struct SortBufs {
     void *slot = nullptr;
     unsigned long long *jobq = nullptr;  // [kJobqWords] SM job queue words, zero between launches
     void *scan_part = nullptr;  // int2[ceil(nbins / chunk)]
+    // window kernels: the current points' window order (see WinPts)
+    WinGeom win;
+    int *wcount = nullptr;     // [nkeys] zero between setpts calls
+    int *wstart = nullptr;     // [nkeys + 1]
+    int *wused = nullptr;      // [nkeys + 1] windows with points before each
+    void *wpart = nullptr;     // scan partials (int2) and totals
+    int *wrange = nullptr;     // [ranges + 1]
+    void *wx = nullptr;        // T [dim][pos_stride]
+    unsigned *wsh = nullptr;   // [M]
+    int *widx = nullptr;       // [M]
     // method 4: point copies counted per block
     int *kcount = nullptr;       // [nkeys]
     int *kstart = nullptr;       // [nkeys]
@@ -120,6 +155,31 @@ template <typename T>
 int run_interp(int method, int dim, int ns, int M, const SortBufs &sb, cpx<T> *c,
                const cpx<T> *fw, const BinGeom &g, const KerParams<T> &kp, int maxsub,
                long long sub_bound, int ntr, long long nftot, const Launch &L);
+
+// Window kernels: kernel widths built (3D FP64 spreads hold ns planes of 16 x 16
+// complex cells in registers, which ends at 13).
+constexpr bool win_spread_width(int, int ns, size_t elem)
+{
+    return ns >= 4 && ns <= (elem == 4 ? 9 : 13);
+}
+constexpr bool win_interp_width(int, int ns, size_t elem)
+{
+    return ns >= 4 && ns <= (elem == 4 ? 9 : 13);
+}
+// Windows for M points (ranges = 0 where the per-point kernels are the better
+// ones), and the window order of the points after run_bin_sort.
+WinGeom win_choose(int type, int dim, int ns, int elem, const BinGeom &g, int M, int ntr, int ncu);
+int run_win_clear(const SortBufs &sb, long long keys, const Launch &L);  // wcount = 0
+template <typename T>
+int run_win_sort(int dim, int M, const SortBufs &sb, const Launch &L);
+template <typename T, int DIM>
+int win_spread_dim(int ns, int M, const SortBufs &sb, const cpx<T> *c, cpx<T> *fw,
+                   const BinGeom &g, const KerParams<T> &kp, int ntr, long long nftot,
+                   const Launch &L);
+template <typename T, int DIM>
+int win_interp_dim(int ns, int M, const SortBufs &sb, cpx<T> *c, const cpx<T> *fw,
+                   const BinGeom &g, const KerParams<T> &kp, int ntr, long long nftot,
+                   const Launch &L);
 
 // Cells of the SM tile of a bin: the bin plus a halo of ceil(ns/2) per side.
 inline size_t sm_tile_cells(int dim, int ns, const int *bs)

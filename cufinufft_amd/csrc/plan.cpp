@@ -542,6 +542,7 @@ struct Plan {
         dfree(sb.jobq);
         if (sb.scan_part) hipFree(sb.scan_part);
         sb.scan_part = nullptr;
+        free_win();
         dfree(sb.kcount);
         dfree(sb.kstart);
         if (sb.kscan_part) hipFree(sb.kscan_part);
@@ -714,6 +715,22 @@ struct Plan {
     int setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned char *scr,
                        size_t scr_bytes);
     int setpts_blocks();
+    WinGeom choose_win(int M_) const;
+    long long cap_wkeys = -1, cap_wM = -1, cap_wranges = -1;  // of the window order
+    int alloc_win();
+    void free_win()
+    {
+        dfree(sb.wcount);
+        dfree(sb.wstart);
+        dfree(sb.wused);
+        dfree(sb.wrange);
+        if (sb.wpart) hipFree(sb.wpart);
+        if (sb.wx) hipFree(sb.wx);
+        sb.wpart = sb.wx = nullptr;
+        dfree(sb.wsh);
+        dfree(sb.widx);
+        cap_wkeys = cap_wM = cap_wranges = -1;
+    }
     int cap_copies = -1;  // capacity of idx / pos in point copies (method 4)
     long long cap_counts = -1;          // capacity of sb.sort_counts
     long long cap_rec[2] = {-1, -1};    // capacity of sb.rec[] in points
@@ -1042,6 +1059,41 @@ int Plan<T>::setpts_blocks()
     return 0;
 }
 
+// Windows of the window kernels, or ranges = 0 for the per-point ones.
+template <typename T>
+WinGeom Plan<T>::choose_win(int M_) const
+{
+    if (dim < 2 || method == 4 || (method == 1 && (!opts.gpu_sort || type == 1))) return WinGeom();
+    if (type == 2 && opts.gpu_spreadinterponly) return WinGeom();
+    return win_choose(type, dim, sp.ns, sizeof(T), geom, M_, ntransf, L.ncu);
+}
+
+// Arrays of the window order for sb.win (grown on demand; x as the positions,
+// cap_M points per axis).
+template <typename T>
+int Plan<T>::alloc_win()
+{
+    const long long keys = sb.win.nkeys;
+    if (keys <= cap_wkeys && M <= cap_wM && sb.win.ranges <= cap_wranges) return 0;
+    free_win();
+    const long long parts = (keys + kScanChunk - 1) / kScanChunk;
+    if (dmalloc(&sb.wcount, (size_t)keys) || dmalloc(&sb.wstart, (size_t)keys + 1) ||
+        dmalloc(&sb.wused, (size_t)keys + 1) ||
+        hipMalloc(&sb.wpart, sizeof(int2) * (size_t)(parts + 1)) != hipSuccess ||
+        dmalloc(&sb.wrange, (size_t)sb.win.ranges + 1) ||
+        hipMalloc(&sb.wx, sizeof(T) * (size_t)sb.pos_stride * dim) != hipSuccess ||
+        dmalloc(&sb.wsh, (size_t)sb.pos_stride) || dmalloc(&sb.widx, (size_t)sb.pos_stride) ||
+        run_win_clear(sb, keys, L)) {
+        (void)hipGetLastError();
+        free_win();
+        return kErrHip;
+    }
+    cap_wkeys = keys;
+    cap_wranges = sb.win.ranges;
+    cap_wM = sb.pos_stride;
+    return 0;
+}
+
 template <typename T>
 int Plan<T>::setpts(int M_, const T *x, const T *y, const T *z)
 {
@@ -1107,6 +1159,9 @@ int Plan<T>::setpts(int M_, const T *x, const T *y, const T *z)
         }
         cap_sub = sub_bound;
     }
+    sb.win = choose_win(M);
+    // without memory for the window order the per-point kernels run
+    if (sb.win.ranges > 0 && alloc_win()) sb.win = WinGeom();
     int e;
     {
         Stage st(this, kStageSort);
@@ -1116,6 +1171,7 @@ int Plan<T>::setpts(int M_, const T *x, const T *y, const T *z)
             e = run_bin_sort<T>(dim, geom, nbins, M, kx, ky, kz, maxsub, opts.gpu_sort == 2,
                                 need_sub, sb, L);
         }
+        if (!e && sb.win.ranges > 0) e = run_win_sort<T>(dim, M, sb, L);
     }
     if (e) return e;
     pts_set = true;
@@ -1142,6 +1198,9 @@ int Plan<T>::setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned
     const long long sub_need = nbins + (M_ + (long long)maxsub - 1) / maxsub;
     const bool need_sub = method == 2;
     if (need_sub && sub_need > cap_sub) return kErrNoAlloc;
+    // the window order needs its arrays too: without them the per-point kernels run
+    WinGeom win = choose_win(M_);
+    if (win.nkeys > cap_wkeys || M_ > cap_wM || win.ranges > cap_wranges) win = WinGeom();
     SortBufs s2 = sb;
     if (!(method == 1 && !opts.gpu_sort) && M_ > 0) {
         const long long nkeys =
@@ -1169,6 +1228,7 @@ int Plan<T>::setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned
     ky = dim > 1 ? y : nullptr;
     kz = dim > 2 ? z : nullptr;
     sub_bound = sub_need;
+    sb.win = win;
     int e;
     {
         Stage st(this, kStageSort);
@@ -1178,6 +1238,7 @@ int Plan<T>::setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned
             e = run_bin_sort<T>(dim, geom, nbins, M, kx, ky, kz, maxsub, opts.gpu_sort == 2,
                                 need_sub, s2, L);
         }
+        if (!e && sb.win.ranges > 0) e = run_win_sort<T>(dim, M, sb, L);
     }
     pts_set = e == 0;
     return e;

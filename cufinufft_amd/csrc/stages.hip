@@ -114,6 +114,9 @@ int run_spread(int method, int dim, int ns, int M, const SortBufs &sb, const cpx
                long long sub_bound, int ntr, long long nftot, const Launch &L)
 {
     if (M == 0) return 0;
+    if (sb.win.ranges > 0)
+        return dim == 2 ? win_spread_dim<T, 2>(ns, M, sb, c, fw, g, kp, ntr, nftot, L)
+                        : win_spread_dim<T, 3>(ns, M, sb, c, fw, g, kp, ntr, nftot, L);
     if (dim == 1)
         return spread_dim<T, 1>(method, ns, M, sb, c, fw, g, kp, maxsub, sub_bound, ntr, nftot, L);
     if (dim == 2)
@@ -127,6 +130,9 @@ int run_interp(int method, int dim, int ns, int M, const SortBufs &sb, cpx<T> *c
                long long sub_bound, int ntr, long long nftot, const Launch &L)
 {
     if (M == 0) return 0;
+    if (sb.win.ranges > 0)
+        return dim == 2 ? win_interp_dim<T, 2>(ns, M, sb, c, fw, g, kp, ntr, nftot, L)
+                        : win_interp_dim<T, 3>(ns, M, sb, c, fw, g, kp, ntr, nftot, L);
     if (dim == 1)
         return interp_dim<T, 1>(method, ns, M, sb, c, fw, g, kp, maxsub, sub_bound, ntr, nftot, L);
     if (dim == 2)

@@ -1,0 +1,686 @@
+// Window kernels: spreading and interpolation in 2D and 3D as small matrix
+// products on the matrix cores (v_mfma_{f32_16x16x4f32, f64_16x16x4f64}).
+//
+// The ns^DIM taps of a point are an outer product of its axis weights, so the
+// taps of many points that share a small window of the fine grid form a
+// matrix product over the points:
+//   spread:  win[(y, z), x] += sum_p (ky_p[y] kz_p[z]) * (c_p kx_p[x])
+//   interp:  g[p, x] = sum_(y, z) (ky_p[y] kz_p[z]) * win[(y, z), x],
+//            c_p = sum_x kx_p[x] g[p, x]
+// with weights that are 0 outside a point's own taps.  A window is 16 cells
+// wide in x, so it holds every point whose first tap lies in its first 17 - ns
+// cells, and likewise along the other axes.  setpts orders the points by window
+// (win_sort.hip); a wave then takes a range of that order and keeps a whole
+// window in registers, so a tap costs neither an LDS operation nor a VALU
+// instruction of its own.  No wave waits for another.
+//
+// What this replaces was bound by exactly those: the per-point spread issued
+// two LDS atomics and six VALU instructions per tap (14 / 10 / 7 lanes per
+// clock and CU for 32-bit, 64-bit integer and FP64 LDS adds), the per-point
+// interp one LDS or L1 read and two FMAs per tap.
+// Spread or interp alone, per-point -> window kernel: 3D FP32 type 1, ns 6, 1e8
+// points on 512^3: 20.7 -> 7.9 ms; 3D FP64 type 2, ns 10, 1e7: 17.7 -> 3.4 ms;
+// 2D FP64 type 2: 0.90 -> 0.39 ms (the rule of win_sort.hip has both sides at
+// the edges of its range).
+#pragma once
+#include <utility>
+
+#include "nufft_device.cuh"
+
+namespace cfa {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+template <typename T> struct Mfma;
+template <> struct Mfma<float> {
+    using Acc = v4f;
+    __device__ static __forceinline__ Acc mac(float a, float b, Acc c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+};
+template <> struct Mfma<double> {
+    using Acc = v4d;
+    __device__ static __forceinline__ Acc mac(double a, double b, Acc c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+};
+
+// Row of the 16 x 16 result held by register r of the lanes of quarter q
+// (the column is the lane within the quarter).
+template <typename T>
+__device__ __forceinline__ int mfma_row(int q, int r)
+{
+    return sizeof(T) == 4 ? 4 * q + r : q + 4 * r;
+}
+
+// Lane movement inside rows of 16 lanes (DPP); CTRL as in the ISA's dpp_ctrl:
+// 0x150 + n broadcasts lane n of each row, 0x120 + n rotates right by n, 0x100 +
+// n / 0x110 + n shift by n lanes down / up, 0x55 n broadcasts lane n of each quad.
+// Lanes whose bank (4 lanes) is not in BANKS keep old.
+template <int CTRL, int BANKS>
+__device__ __forceinline__ float dpp(float old, float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL,
+                                                      0xf, BANKS, false));
+}
+template <int CTRL, int BANKS>
+__device__ __forceinline__ double dpp(double old, double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf,
+                                               BANKS, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf,
+                                               BANKS, false);
+    return __hiloint2double(hi, lo);
+}
+constexpr int kDppBcast = 0x150, kDppRor = 0x120, kDppShl = 0x100, kDppShr = 0x110;
+
+// f(0), ..., f(N - 1) with the index as a compile-time constant.
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Sum over each row of 16 lanes, in every lane.
+template <typename T>
+__device__ __forceinline__ T row_sum(T v)
+{
+    v += dpp<kDppRor + 8, 0xf>(v, v);
+    v += dpp<kDppRor + 4, 0xf>(v, v);
+    v += dpp<kDppRor + 2, 0xf>(v, v);
+    v += dpp<kDppRor + 1, 0xf>(v, v);
+    return v;
+}
+
+// Square root of a in [2^-60, 1], within an ulp: the hardware reciprocal square
+// root and Newton (Goldschmidt) steps with fused residuals.  The library's
+// sqrt spends most of its instructions on ranges that cannot occur here.
+__device__ __forceinline__ double win_sqrt(double a)
+{
+    const double y = __builtin_amdgcn_rsq(a);
+    double s = a * y, h = 0.5 * y;
+    const double r = fma(-h, s, 0.5);
+    s = fma(s, r, s);
+    h = fma(h, r, h);
+    return fma(fma(-s, s, a), h, s);
+}
+
+// e^x in FP64 for |x| < 700: x = n ln 2 + r with |r| <= ln 2 / 2 (ln 2 in two
+// parts), the Taylor polynomial of e^r to r^13 (its remainder is 4e-18), and a
+// scaling by 2^n.
+__device__ __forceinline__ double win_exp(double x)
+{
+    const double n = __builtin_rint(x * 1.4426950408889634);
+    double r = fma(n, -0x1.62e42fefa3800p-1, x);
+    r = fma(n, -0x1.ef35793c76730p-45, r);
+    double p = 1.0 / 6227020800.0;
+    p = fma(p, r, 1.0 / 479001600.0);
+    p = fma(p, r, 1.0 / 39916800.0);
+    p = fma(p, r, 1.0 / 3628800.0);
+    p = fma(p, r, 1.0 / 362880.0);
+    p = fma(p, r, 1.0 / 40320.0);
+    p = fma(p, r, 1.0 / 5040.0);
+    p = fma(p, r, 1.0 / 720.0);
+    p = fma(p, r, 1.0 / 120.0);
+    p = fma(p, r, 1.0 / 24.0);
+    p = fma(p, r, 1.0 / 6.0);
+    p = fma(p, r, 0.5);
+    p = fma(p, r, 1.0);
+    p = fma(p, r, 1.0);
+    return __builtin_ldexp(p, (int)n);
+}
+
+// Kernel value at offset x from the point, over its peak: phi(x) / e^beta; the
+// callers put e^(DIM beta) back in FP64.  Outside the support, and for ok =
+// false, the exponent is replaced by one that underflows to 0, so the code has
+// no branch: many evaluations overlap.
+//
+// FP32 forms the exponent beta (sqrt(1 - t) - 1), t = c x^2, as -beta t /
+// (1 + sqrt(1 - t)): its rounding is then relative to the exponent, which is
+// small where the kernel is large, and the hardware square root and reciprocal
+// (1 ulp) do.  The difference sqrt(..) - 1 itself carries half an ulp of 1, times
+// beta (14 - 20) a relative error of ~3e-7 in every weight.
+__device__ __forceinline__ float win_phi(float x, const KerParams<float> &k, bool ok = true)
+{
+    const float t = k.c * x * x;
+    const float s = __builtin_amdgcn_sqrtf(fmaxf(1.0f - t, 0.0f));
+    const float w = t * __builtin_amdgcn_rcpf(1.0f + s);
+    const float e = fmaf(-k.bl2e, w, -k.bl2e_lo * w);
+    return __builtin_amdgcn_exp2f(((fabsf(x) < k.hw) & ok) ? e : -1000.0f);
+}
+__device__ __forceinline__ double win_phi(double x, const KerParams<double> &k, bool ok = true)
+{
+    const double v = win_exp(k.beta * (win_sqrt(fmax(1.0 - k.c * x * x, 0x1p-60)) - 1.0));
+    return ((fabs(x) < k.hw) & ok) ? v : 0.0;
+}
+
+// Place of a point (position v, in [-1, nf + 1]) along one axis: its first tap
+// is cell u - P - 1, u >= 0; f = first tap - position + ns/2 in [0, 1).  The weight
+// of tap i is evaluated at f + (i - ns/2): i - ns/2 is exact, so a point keeps the
+// precision of f, 2^-25 in FP32 (first tap - position itself would round at 2^-23).
+// Window k of S first taps starts at cell k S - P - 1.
+CFA_HD int win_first(int ns) { return (ns + 1) / 2 + 1; }
+template <typename T>
+CFA_HD int win_place(double v, int ns, T &f)
+{
+    const double s = ceil(v - 0.5 * ns);
+    f = (T)((s - v) + 0.5 * ns);
+    return (int)s + win_first(ns);
+}
+// Grid index of a cell in [-nf, 2 nf).
+CFA_HD int win_wrap(int c, int n)
+{
+    c += c < 0 ? n : 0;
+    return c - (c >= n ? n : 0);
+}
+
+// Key of a window: along z (3D) fastest, then x, then y, so a strip of windows
+// along z is a run of the order.
+template <int DIM>
+CFA_HD int win_key(const WinGeom &w, const int *k)
+{
+    return DIM == 3 ? (k[1] * w.nw[0] + k[0]) * w.nw[2] + k[2] : k[1] * w.nw[0] + k[0];
+}
+
+// Windows of a grid nf for transforms of the given type and width: S, nw, nkeys,
+// ns.  false: a grid so small that a window's cells could wrap twice, or too
+// many windows to count in ints.
+inline bool win_windows(int type, int dim, int ns, const int *nf, WinGeom &w)
+{
+    w.ns = ns;
+    w.S[0] = w.S[1] = 17 - ns;
+    w.S[2] = 1;
+    if (dim == 3 && type == 2) w.S[1] = w.S[2] = 2 * win_interp_half(ns) - ns + 1;
+    double keys = 1;
+    for (int d = 0; d < dim; ++d) {
+        if (nf[d] < 24) return false;
+        w.nw[d] = (nf[d] + 3) / w.S[d] + 1;
+        keys *= w.nw[d];
+    }
+    if (keys > 1 << 27) return false;
+    w.nkeys = (int)keys;
+    return true;
+}
+
+// First point of range r of `ranges` ranges of equal weight, a point counting 1
+// and a window that has points kWinKeyWeight (before its points).  start and used:
+// points and windows with points before each key (used[nkeys]: all).
+CFA_HD int win_range_start(const int *start, const int *used, int nkeys, int M, int r, int ranges)
+{
+    if (r >= ranges) return M;
+    const long long total = M + (long long)kWinKeyWeight * used[nkeys];
+    const long long w = total * r / ranges;
+    int lo = 0, hi = nkeys - 1;  // last key whose weight starts at or before w
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (start[mid] + (long long)kWinKeyWeight * used[mid] <= w) lo = mid; else hi = mid - 1;
+    }
+    const long long off = w - start[lo] - (long long)kWinKeyWeight * (used[lo] + 1);
+    const int n = (lo + 1 < nkeys ? start[lo + 1] : M) - start[lo];
+    return start[lo] + (int)(off > 0 ? (off < n ? off : n) : 0);
+}
+
+// Last key k with start[k] <= p (n keys): the key of point p.
+__device__ __forceinline__ int win_key_of(const int *__restrict__ start, int n, int p)
+{
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (start[mid] <= p) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+// The keys of a wave's range, in order: 64 of their ends in the lanes.
+struct WinKeys {
+    int base, end;  // lane j: start[base + 1 + j]
+    __device__ __forceinline__ void load(const WinPts &wp, int nkeys, int key)
+    {
+        base = key;
+        end = wp.start[min(key + 1 + (int)(threadIdx.x & 63), nkeys)];
+    }
+    // Key of point p (>= the points asked for before).
+    __device__ __forceinline__ int key_of(const WinPts &wp, int nkeys, int p)
+    {
+        unsigned long long m = __ballot(end > p);
+        if (!m) {  // past these 64: a run of empty keys, or the next ones
+            int k = base + 64;
+            if (wp.start[min(k + 64, nkeys)] <= p) k = win_key_of(wp.start, nkeys, p);
+            load(wp, nkeys, k);
+            m = __ballot(end > p);
+        }
+        return base + __builtin_ctzll(m);
+    }
+    __device__ __forceinline__ int key_end(int key) const
+    {
+        return __builtin_amdgcn_readlane(end, key - base);
+    }
+};
+
+// A staged point in LDS.
+template <typename T>
+struct alignas(4 * sizeof(T)) WinRec {
+    T x[3];
+    unsigned sh;  // first tap inside its window, a byte per axis
+};
+
+// ---------------------------------------------------------------------------
+// Spread.  Windows of 16 x 16 cells in (x, y).  In 3D the points of a strip
+// of windows come in order of their first z plane; the registers hold the ns
+// planes that the current first plane reaches, plane z in slot z mod ns, and
+// when the first plane moves on, the planes left behind go to the fine grid
+// with global atomics.  So a strip writes every cell of its 16 x 16 column
+// once: 256 / (17 - ns)^2 cells per grid cell (2.1 at ns 6), and no LDS tile, no
+// common scale and no barrier is needed.  In 2D a window is one such plane,
+// and NT transforms share the weights.
+//
+// Bounds per point (rate of a CU): 4 ns (FP32) or 8 ns clocks of the matrix
+// cores in 3D, about 20 VALU instructions for the weights, and the atomics, at
+// 3.0e11 (FP32) or 1.75e11 (FP64) lanes per second on the whole device.
+template <typename T, int DIM, int NS, int NT>
+struct WinSpread {
+    using Acc = typename Mfma<T>::Acc;
+    static constexpr int RB = DIM == 3 ? NS : 1;
+    Acc ar[NT][RB], ai[NT][RB];
+    unsigned row[4], col[2];  // see place()
+
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int m = 0; m < RB; ++m) ar[t][m] = ai[t][m] = Acc{0, 0, 0, 0};
+    }
+    // The window's place (kx, ky): where in a plane the components go that
+    // flush() hands this lane.
+    __device__ __forceinline__ void place(int kx, int ky, const BinGeom &g)
+    {
+        constexpr int S = 17 - NS, F = (NS + 1) / 2 + 1;
+        const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            row[r] = 2u * (unsigned)(win_wrap(ky * S - F + mfma_row<T>(q, r), g.nf[1]) * g.nf[0]);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            col[b] = 2u * (unsigned)win_wrap(kx * S - F + 8 * b + (i16 >> 1), g.nf[0]) + (i16 & 1);
+    }
+    // Points s .. e - 1 of the staged batch (of one window); zslot: slot of
+    // their first plane.
+    __device__ __forceinline__ void accumulate(int s, int e, int zslot, const WinRec<T> *rec,
+                                               const cpx<T> *cs, const KerParams<T> &kp)
+    {
+        const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
+        // lane i of a row evaluates the x and y weights of cell i and the z
+        // weight of slot i
+        const T hw = T(0.5) * NS, f = (T)i16 - hw;
+        const int zt = i16 - zslot;
+        const T fz = (T)(zt < 0 ? zt + NS : zt) - hw;
+        for (int b = s; b < e; b += 4) {
+            // quarter q of the wave holds point b + q
+            const bool ok = b + q < e;
+            const int p = ok ? b + q : s;
+            const WinRec<T> r = rec[p];
+            const T kx = win_phi(r.x[0] + (f - (T)(r.sh & 255)), kp, ok);
+            const T ky = win_phi(r.x[1] + (f - (T)(r.sh >> 8 & 255)), kp);
+            T kz = T(0);
+            if (DIM == 3) kz = win_phi(r.x[2] + fz, kp);
+            T br[NT], bi[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const cpx<T> v = cs[64 * t + p];
+                br[t] = v.x * kx;
+                bi[t] = v.y * kx;
+            }
+            static_for<RB>([&](auto mc) {
+                constexpr int m = decltype(mc)::value;
+                const T a = DIM == 3 ? ky * dpp<kDppBcast + m, 0xf>(kz, kz) : ky;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    ar[t][m] = Mfma<T>::mac(a, br[t], ar[t][m]);
+                    ai[t][m] = Mfma<T>::mac(a, bi[t], ai[t][m]);
+                }
+            });
+        }
+    }
+    // Adds plane slot m of every transform to the grid and clears it; plane: the
+    // plane's first cell in transform 0.  The lanes first trade places through
+    // LDS (sc, 256 complex values of the wave), so that 16 lanes add the 16
+    // components of 8 neighbouring cells: 1.9e11 adds per second against 1.2e11
+    // for a lane per cell that adds its two components in turn (16 x 16 windows
+    // every 10 cells of a 1024^2 FP32 grid).
+    template <int m>
+    __device__ __forceinline__ void flush(T *plane, long long tstride, int nt, cpx<T> *sc)
+    {
+        const int lane = threadIdx.x & 63;
+        const T *src = reinterpret_cast<const T *>(sc) + (lane & 48) * 2 + (lane & 15);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if (NT == 1 || t < nt) {
+                T *p = plane + t * tstride;
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    cpx<T> v;
+                    v.x = ar[t][m][r];
+                    v.y = ai[t][m][r];
+                    sc[64 * r + lane] = v;
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const T v = src[128 * r + 16 * b];
+                        if (v != T(0)) gadd(p + (row[r] + col[b]), v);
+                    }
+            }
+            ar[t][m] = ai[t][m] = Acc{0, 0, 0, 0};
+        }
+    }
+};
+
+template <typename T, int DIM, int NS, int NT>
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
+k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict__ fw, BinGeom g,
+             WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
+{
+    constexpr int F = (NS + 1) / 2 + 1;
+    __shared__ WinRec<T> srec[256];
+    __shared__ cpx<T> scs[256 * NT], ssc[1024];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    WinRec<T> *rec = srec + wave * 64;
+    cpx<T> *cs = scs + wave * 64 * NT, *sc = ssc + wave * 256;
+    const T *x1 = static_cast<const T *>(wp.x);
+    const JobRange jr = xcd_jobs(gridDim.x);  // one range per wave, contiguous per XCD
+    const int rng = (int)jr.begin * 4 + wave;
+    if (rng >= wg.ranges) return;
+    int p = wp.range[rng];
+    const int pe = wp.range[rng + 1];
+    if (p >= pe) return;
+    const int t0 = blockIdx.y * NT, nt = min(NT, ntr - t0);
+    c += (long long)t0 * M;
+    T *ft = reinterpret_cast<T *>(fw + (long long)t0 * nftot);
+    const double back = exp((double)DIM * (double)kp.beta);
+    WinSpread<T, DIM, NS, NT> acc;
+    acc.clear();
+    WinKeys keys;
+    keys.load(wp, wg.nkeys, win_key_of(wp.start, wg.nkeys, p));
+    // batches of 64 points, one per lane: the next batch's strengths and the
+    // records of the one after are in flight while one is worked on
+    T xa[DIM], xb[DIM];
+    unsigned sa, sb;
+    int ib;
+    cpx<T> ca[NT];
+    auto load = [&](int i, T *x, unsigned &s, int &id) {
+        const int k = min(i, pe - 1);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) x[d] = x1[d * wp.stride + k];
+        s = wp.sh[k];
+        id = wp.idx[k];
+    };
+    auto gather = [&](int id) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            ca[t].x = ca[t].y = T(0);
+            if (NT == 1 || t < nt) ca[t] = c[(long long)t * M + id];
+        }
+    };
+    load(p + lane, xa, sa, ib);
+    gather(ib);
+    load(p + 64 + lane, xb, sb, ib);
+    int b0 = p;
+    bool staged = false;
+    int strip = -1, z = 0;  // window held (3D: its first plane's place too)
+    const int nz = DIM == 3 ? wg.nw[2] : 1;
+    const long long pstride = 2ll * g.nf[0] * g.nf[1];
+    for (;;) {
+        const bool last = p >= pe;
+        int key = 0, ke = 0, st = -1, zk = 0;
+        if (!last) {
+            key = keys.key_of(wp, wg.nkeys, p);
+            ke = min(pe, keys.key_end(key));
+            st = DIM == 3 ? key / nz : key;
+            zk = DIM == 3 ? key - st * nz : 0;
+        }
+        // the planes no later point of the strip reaches go to the grid
+        const int nf = strip < 0 ? 0 : (st != strip ? acc.RB : min(zk - z, acc.RB));
+        for (int k = z; k < z + nf; ++k) {
+            T *plane = ft + (DIM == 3 ? win_wrap(k - F, g.nf[2]) * pstride : 0);
+            const int m = DIM == 3 ? k % NS : 0;
+            static_for<WinSpread<T, DIM, NS, NT>::RB>([&](auto mc) {
+                if (m == decltype(mc)::value)
+                    acc.template flush<decltype(mc)::value>(plane, 2 * nftot, nt, sc);
+            });
+        }
+        if (last) break;
+        if (st != strip) acc.place(st % wg.nw[0], st / wg.nw[0], g);
+        strip = st;
+        z = zk;
+        while (p < ke) {
+            if (!staged || p >= b0 + 64) {
+                if (staged) b0 += 64;
+                staged = true;
+                __builtin_amdgcn_wave_barrier();
+                WinRec<T> r;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) r.x[d] = xa[d];
+                r.sh = sa;
+                rec[lane] = r;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    ca[t].x = (T)((double)ca[t].x * back);
+                    ca[t].y = (T)((double)ca[t].y * back);
+                    cs[64 * t + lane] = ca[t];
+                }
+                gather(ib);
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) xa[d] = xb[d];
+                sa = sb;
+                load(b0 + 128 + lane, xb, sb, ib);
+                __builtin_amdgcn_wave_barrier();
+            }
+            const int e = min(ke, b0 + 64);
+            acc.accumulate(p - b0, e - b0, DIM == 3 ? z % NS : 0, rec, cs, kp);
+            p = e;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Interp (the product's inner dimension = (y, z) cells, 4 per instruction,
+// one for each quarter of the wave).  3D: quarter (a, b) holds the y cells
+// a HY .. and z cells b HZ ..; 2D: quarter q holds y = 4 i + q.  A wave takes
+// up to NB batches of 16 points of one window: it evaluates their y and z
+// weights in the operand layout of the product (each lane only those of its
+// own cells), reads the window's cells straight from the fine grid (a window is
+// read once per run; neighbouring windows share lines in L1 and L2) and
+// finishes with the x weights and a sum over 16 lanes.
+template <int DIM, int NS>
+struct InterpWin {
+    static constexpr int NB = DIM == 3 ? 2 : 4;
+    static constexpr int HY = DIM == 2 ? 4 : win_interp_half(NS);
+    static constexpr int HZ = DIM == 2 ? 1 : HY;
+    static constexpr int SX = 17 - NS, SY = DIM == 2 ? 17 - NS : 2 * HY - NS + 1,
+                         SZ = DIM == 2 ? 1 : 2 * HZ - NS + 1;
+};
+
+template <typename T, int DIM, int NS, int NB>
+__device__ __forceinline__ void win_interp_run(int s, int npt, int gx, const int *yo,
+                                               const long long *zo, int M, int ntr,
+                                               cpx<T> *__restrict__ c,
+                                               const cpx<T> *__restrict__ fw, long long nftot,
+                                               const KerParams<T> &kp, double back,
+                                               const WinRec<T> *rec, const int *ids)
+{
+    using W = InterpWin<DIM, NS>;
+    using Acc = typename Mfma<T>::Acc;
+    const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
+    const T hw = T(0.5) * NS;
+    T ky[NB][W::HY], kz[NB][W::HZ], kx[NB][4];
+    int dst[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const WinRec<T> r = rec[s + min(16 * b + i16, npt - 1)];
+        const T fy = (T)(DIM == 2 ? q : (q & 1) * W::HY) - hw - (T)(r.sh >> 8 & 255);
+#pragma unroll
+        for (int k = 0; k < W::HY; ++k)
+            ky[b][k] = win_phi(r.x[1] + (fy + (T)(DIM == 2 ? 4 * k : k)), kp);
+        if (DIM == 3) {
+            const T fz = (T)((q >> 1) * W::HZ) - hw - (T)(r.sh >> 16 & 31);
+#pragma unroll
+            for (int k = 0; k < W::HZ; ++k) kz[b][k] = win_phi(r.x[2] + (fz + (T)k), kp);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const WinRec<T> &rk = rec[s + min(16 * b + mfma_row<T>(q, k), npt - 1)];
+            kx[b][k] = win_phi(rk.x[0] + ((T)i16 - hw - (T)(rk.sh & 255)), kp);
+        }
+        // the lanes i16 < 4 of quarter q store the point of result row i16
+        const int pd = 16 * b + mfma_row<T>(q, i16 & 3);
+        dst[b] = i16 < 4 && pd < npt ? ids[s + pd] : -1;
+    }
+    for (int t = 0; t < ntr; ++t) {
+        const cpx<T> *f = fw + (long long)t * nftot + gx;
+        // keep the ky kz products inside the loop over transforms (hoisted
+        // out of it they would take HY HZ registers per batch)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int k = 0; k < W::HY; ++k) asm volatile("" : "+v"(ky[b][k]));
+        Acc ar[NB], ai[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) ar[b] = ai[b] = Acc{0, 0, 0, 0};
+        // one plane of cells in flight while the one before is multiplied
+        cpx<T> v[2][W::HY];
+#pragma unroll
+        for (int k = 0; k < W::HY; ++k) v[0][k] = f[(DIM == 3 ? zo[0] : 0) + yo[k]];
+#pragma unroll
+        for (int kk = 0; kk < W::HZ; ++kk) {
+            if (kk + 1 < W::HZ)
+#pragma unroll
+                for (int k = 0; k < W::HY; ++k) v[(kk + 1) & 1][k] = f[zo[kk + 1] + yo[k]];
+#pragma unroll
+            for (int k = 0; k < W::HY; ++k)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const T a = DIM == 3 ? ky[b][k] * kz[b][kk] : ky[b][k];
+                    ar[b] = Mfma<T>::mac(a, v[kk & 1][k].x, ar[b]);
+                    ai[b] = Mfma<T>::mac(a, v[kk & 1][k].y, ai[b]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            cpx<T> o;
+            o.x = o.y = T(0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const T sr = row_sum(ar[b][k] * kx[b][k]), si = row_sum(ai[b][k] * kx[b][k]);
+                o.x = i16 == k ? sr : o.x;
+                o.y = i16 == k ? si : o.y;
+            }
+            o.x = (T)((double)o.x * back);
+            o.y = (T)((double)o.y * back);
+            if (dst[b] >= 0) c[(long long)t * M + dst[b]] = o;
+        }
+    }
+}
+
+// Workgroups of 4 independent waves, one range of the order each; each XCD takes
+// a contiguous part of it.
+template <typename T, int DIM, int NS>
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
+k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict__ fw, BinGeom g,
+             WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
+{
+    using W = InterpWin<DIM, NS>;
+    constexpr int F = (NS + 1) / 2 + 1;
+    __shared__ WinRec<T> srec[256];
+    __shared__ int sids[256];
+    const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    WinRec<T> *rec = srec + wave * 64;
+    int *ids = sids + wave * 64;
+    const T *x1 = static_cast<const T *>(wp.x);
+    const JobRange jr = xcd_jobs(gridDim.x);
+    const int rng = (int)jr.begin * 4 + wave;
+    if (rng >= wg.ranges) return;
+    int p = wp.range[rng];
+    const int pe = wp.range[rng + 1];
+    if (p >= pe) return;
+    const double back = exp((double)DIM * (double)kp.beta);
+    WinKeys keys;
+    keys.load(wp, wg.nkeys, win_key_of(wp.start, wg.nkeys, p));
+    T xa[DIM];
+    unsigned sa;
+    int ia;
+    auto load = [&](int i) {
+        const int k = min(i, pe - 1);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) xa[d] = x1[d * wp.stride + k];
+        sa = wp.sh[k];
+        ia = wp.idx[k];
+    };
+    load(p + lane);
+    int b0 = p;
+    bool staged = false;
+    while (p < pe) {
+        const int key = keys.key_of(wp, wg.nkeys, p);
+        const int ke = min(pe, keys.key_end(key));
+        const int st = DIM == 3 ? key / wg.nw[2] : key;
+        const int kz = DIM == 3 ? key - st * wg.nw[2] : 0;
+        const int ky = st / wg.nw[0], kx = st - ky * wg.nw[0];
+        // the window's cells of this lane on the periodic grid
+        const int gx = win_wrap(kx * W::SX - F + i16, g.nf[0]);
+        int yo[W::HY];
+        long long zo[W::HZ];
+#pragma unroll
+        for (int j = 0; j < W::HY; ++j)
+            yo[j] = win_wrap(ky * W::SY - F + (DIM == 2 ? 4 * j + q : (q & 1) * W::HY + j),
+                             g.nf[1]) *
+                    g.nf[0];
+#pragma unroll
+        for (int j = 0; j < W::HZ; ++j)
+            zo[j] = DIM > 2 ? (long long)win_wrap(kz * W::SZ - F + (q >> 1) * W::HZ + j, g.nf[2]) *
+                                  g.nf[1] * g.nf[0]
+                            : 0;
+        while (p < ke) {
+            if (!staged || p >= b0 + 64) {
+                if (staged) b0 += 64;
+                staged = true;
+                __builtin_amdgcn_wave_barrier();
+                WinRec<T> r;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) r.x[d] = xa[d];
+                r.sh = sa;
+                rec[lane] = r;
+                ids[lane] = ia;
+                load(b0 + 64 + lane);
+                __builtin_amdgcn_wave_barrier();
+            }
+            const int npt = min(min(ke, b0 + 64) - p, 16 * W::NB);
+#define CFA_RUN(NB)                                                                              \
+    win_interp_run<T, DIM, NS, NB>(p - b0, npt, gx, yo, zo, M, ntr, c, fw, nftot, kp, back, rec, \
+                                   ids)
+            if (npt <= 16)
+                CFA_RUN(1);
+            else if (W::NB == 2 || npt <= 32)
+                CFA_RUN(2);
+            else
+                CFA_RUN(W::NB);
+#undef CFA_RUN
+            p += npt;
+        }
+    }
+}
+
+}  // namespace cfa

@@ -1,0 +1,100 @@
+// Runtime-ns dispatch of the window kernels for one (T, DIM); included by the
+// win_spread_<prec><dim>.hip and win_interp_<prec><dim>.hip translation units.
+#include "nufft_launch.h"
+#include "win_device.cuh"
+
+namespace cfa {
+
+namespace {
+
+inline WinPts win_pts(const SortBufs &sb)
+{
+    return WinPts{sb.wx, sb.wsh, sb.widx, sb.wstart, sb.wrange, sb.pos_stride};
+}
+// Workgroups of 4 waves, a range each; whole XCD groups.
+inline int win_grid(const WinGeom &w)
+{
+    const int grid = (w.ranges + 3) / 4;
+    return grid >= kNumXcd ? (grid + kNumXcd - 1) / kNumXcd * kNumXcd : grid;
+}
+
+template <typename T, int DIM, int NS>
+int win_spread_ns(int M, const SortBufs &sb, const cpx<T> *c, cpx<T> *fw, const BinGeom &g,
+                  const KerParams<T> &kp, int ntr, long long nftot, const Launch &L)
+{
+    if constexpr (!win_spread_width(DIM, NS, sizeof(T))) {
+        return 1;
+    } else {
+        const int grid = win_grid(sb.win);
+        if (DIM == 2 && ntr > 1)
+            k_win_spread<T, DIM, NS, DIM == 2 ? 4 : 1>
+                <<<dim3(grid, (ntr + 3) / 4), 256, 0, L.stream>>>(M, win_pts(sb), c, fw, g, sb.win,
+                                                                  kp, ntr, nftot);
+        else
+            k_win_spread<T, DIM, NS, 1><<<dim3(grid, ntr), 256, 0, L.stream>>>(
+                M, win_pts(sb), c, fw, g, sb.win, kp, ntr, nftot);
+        return hipGetLastError() == hipSuccess ? 0 : kErrHip;
+    }
+}
+
+template <typename T, int DIM, int NS>
+int win_interp_ns(int M, const SortBufs &sb, cpx<T> *c, const cpx<T> *fw, const BinGeom &g,
+                  const KerParams<T> &kp, int ntr, long long nftot, const Launch &L)
+{
+    if constexpr (!win_interp_width(DIM, NS, sizeof(T))) {
+        return 1;
+    } else {
+        k_win_interp<T, DIM, NS><<<win_grid(sb.win), 256, 0, L.stream>>>(
+            M, win_pts(sb), c, fw, g, sb.win, kp, ntr, nftot);
+        return hipGetLastError() == hipSuccess ? 0 : kErrHip;
+    }
+}
+
+}  // namespace
+
+#ifndef CFA_NS_CASES
+#define CFA_NS_CASES(F) F(4) F(5) F(6) F(7) F(8) F(9) F(10) F(11) F(12) F(13)
+#endif
+
+template <typename T, int DIM>
+int win_spread_dim(int ns, int M, const SortBufs &sb, const cpx<T> *c, cpx<T> *fw,
+                   const BinGeom &g, const KerParams<T> &kp, int ntr, long long nftot,
+                   const Launch &L)
+{
+    switch (ns) {
+#define CFA_CASE(N)                                                                          \
+    case N:                                                                                  \
+        return win_spread_ns<T, DIM, N>(M, sb, c, fw, g, kp, ntr, nftot, L);
+        CFA_NS_CASES(CFA_CASE)
+#undef CFA_CASE
+    }
+    return 1;
+}
+
+template <typename T, int DIM>
+int win_interp_dim(int ns, int M, const SortBufs &sb, cpx<T> *c, const cpx<T> *fw,
+                   const BinGeom &g, const KerParams<T> &kp, int ntr, long long nftot,
+                   const Launch &L)
+{
+    switch (ns) {
+#define CFA_CASE(N)                                                                          \
+    case N:                                                                                  \
+        return win_interp_ns<T, DIM, N>(M, sb, c, fw, g, kp, ntr, nftot, L);
+        CFA_NS_CASES(CFA_CASE)
+#undef CFA_CASE
+    }
+    return 1;
+}
+
+}  // namespace cfa
+
+#define CFA_INSTANTIATE_WIN_SPREAD(T, DIM)                                                   \
+    template int cfa::win_spread_dim<T, DIM>(int, int, const cfa::SortBufs &,                \
+                                             const cfa::cpx<T> *, cfa::cpx<T> *,             \
+                                             const cfa::BinGeom &, const cfa::KerParams<T> &, \
+                                             int, long long, const cfa::Launch &);
+#define CFA_INSTANTIATE_WIN_INTERP(T, DIM)                                                   \
+    template int cfa::win_interp_dim<T, DIM>(int, int, const cfa::SortBufs &, cfa::cpx<T> *, \
+                                             const cfa::cpx<T> *, const cfa::BinGeom &,      \
+                                             const cfa::KerParams<T> &, int, long long,      \
+                                             const cfa::Launch &);

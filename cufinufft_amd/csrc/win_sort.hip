@@ -1,0 +1,193 @@
+// setpts for the window kernels (win_device.cuh): the rule that chooses them
+// and the order of the points by window.
+//
+// The bin sort leaves the points in bins.  Here they are counted per window and
+// placed in window order, each with what the window kernels need (offsets of the
+// first tap, its place inside the window, the input index), so execute streams 20
+// bytes per 3D FP32 point (28 with positions and index).  A workgroup takes 1024
+// consecutive points of the bin order, which lie in few windows: it counts them
+// in an LDS hash table and does one global atomic per window instead of one per
+// point (random global atomics run at 2e10 per second).
+#include <algorithm>
+
+#include "nufft_launch.h"
+#include "win_device.cuh"
+
+namespace cfa {
+
+constexpr int kWinChunk = 1024;  // points per workgroup
+constexpr int kWinSlots = 2048;  // hash slots: at most half are used
+
+// PLACE = false: count[key] += the points of each key.  PLACE = true: writes
+// the points to start[key] + what is left of count[key], which returns to zero.
+template <typename T, int DIM, bool PLACE>
+__global__ void __launch_bounds__(512)
+k_win_keys(int M, SortedPts sp, WinGeom wg, int *__restrict__ count,
+           const int *__restrict__ start, T *__restrict__ xo, unsigned *__restrict__ sho,
+           int *__restrict__ ido, long long stride)
+{
+    constexpr int BT = 512, PP = kWinChunk / BT;
+    __shared__ int hk[kWinSlots], hc[kWinSlots];
+    const int tid = threadIdx.x;
+    for (int k = tid; k < kWinSlots; k += BT) {
+        hk[k] = -1;
+        hc[k] = 0;
+    }
+    double v[PP][DIM];
+    int id[PP];
+#pragma unroll
+    for (int j = 0; j < PP; ++j) {
+        const int i = min(M - 1, (int)blockIdx.x * kWinChunk + j * BT + tid);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) v[j][d] = sp.pos[d * sp.stride + i];
+        if (PLACE) id[j] = sp.idx[i];
+    }
+    __syncthreads();
+    int slot[PP], rank[PP];
+    unsigned sh[PP];
+    T x1[PP][DIM];
+#pragma unroll
+    for (int j = 0; j < PP; ++j) {
+        slot[j] = -1;
+        if ((int)blockIdx.x * kWinChunk + j * BT + tid >= M) continue;
+        int kw[3] = {0, 0, 0};
+        sh[j] = 0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const int u = win_place<T>(v[j][d], wg.ns, x1[j][d]);
+            kw[d] = u / wg.S[d];
+            sh[j] |= (unsigned)(u - kw[d] * wg.S[d]) << (8 * d);
+        }
+        const int key = win_key<DIM>(wg, kw);
+        unsigned h = (unsigned)key * 2654435761u >> 21;
+        for (;;) {
+            const int old = atomicCAS(&hk[h], -1, key);
+            if (old == -1 || old == key) break;
+            h = (h + 1) & (kWinSlots - 1);
+        }
+        slot[j] = (int)h;
+        rank[j] = atomicAdd(&hc[h], 1);
+    }
+    __syncthreads();
+    for (int k = tid; k < kWinSlots; k += BT) {
+        const int n = hc[k];
+        if (n == 0) continue;
+        if (PLACE)
+            hc[k] = start[hk[k]] + atomicSub(&count[hk[k]], n) - n;
+        else
+            atomicAdd(&count[hk[k]], n);
+    }
+    if (!PLACE) return;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PP; ++j) {
+        if (slot[j] < 0) continue;
+        const int o = hc[slot[j]] + rank[j];
+        sho[o] = sh[j];
+        ido[o] = id[j];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) xo[d * stride + o] = x1[j][d];
+    }
+}
+
+static __global__ void __launch_bounds__(256)
+k_win_ranges(int M, int nkeys, int ranges, int *__restrict__ start, const int *__restrict__ used,
+             int *__restrict__ range)
+{
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r == 0) start[nkeys] = M;
+    if (r <= ranges) range[r] = win_range_start(start, used, nkeys, M, r, ranges);
+}
+
+// Where the window kernels beat the per-point ones, the window order's own time
+// in setpts (30 us, and 15-25 ns per 1000 points) included.  Measured on uniform
+// points, per-point -> window kernel:
+//  3D spread: 0.79 -> 0.29 ms (FP32, ns 6, M = 1e5 on 256^3), 2.3 -> 1.0 ms (1e7),
+//   4.0 -> 0.57 ms (ns 7, 1e6), 14.4 -> 2.8 ms (FP64, ns 10, 1e7); under ~5e4
+//   points (2e4 where the per-point kernel holds 64-bit cells) a window holds so
+//   few points that its flush costs more than their taps, and at ns 4, 5 dense
+//   grids have too few taps per point (0.62 -> 0.68 ms, ns 4, 11 points per cell).
+//  3D interp: a window's cells are read once whatever its points, so it takes
+//   some points per window: 3.1 -> 1.3 ms (FP32, ns 6, 1e7, 59 per window), 0.50
+//   -> 0.58 ms (1e6, 6 per window); FP64 3.0 -> 2.8 ms (ns 10, 4 per window).
+//  2D: few taps, so the order's time decides: 0.65 -> 0.34 ms (FP32, ns 7, 1e7,
+//   order 0.15 ms), 0.078 -> 0.046 ms (1e6, order 0.04 ms); a batch shares it.
+static bool win_pays(int type, int dim, int ns, int elem, int M, int ntr, double per_window)
+{
+    const bool wide = elem == 8 || ns >= 7;
+    if (dim == 3 && type == 1) return M >= (wide ? 20000 : 60000) && (ns >= 6 || elem == 8);
+    if (dim == 3)
+        return M >= 200000 && per_window >= (elem == 8 ? 4 : 8) && (ns >= 6 || elem == 8);
+    const double taps = (double)M * ntr * ns * ns;
+    if (type == 1)
+        return per_window >= 50 && taps >= (elem == 8 ? 1e8 : 2e8) && (ns >= 7 || ntr >= 4);
+    return per_window >= 10 && taps >= (elem == 8 && ns >= 8 ? 1e8 : 4e8) && ns >= 6;
+}
+
+WinGeom win_choose(int type, int dim, int ns, int elem, const BinGeom &g, int M, int ntr, int ncu)
+{
+    WinGeom w, none;
+    if (dim < 2 || M <= 0) return none;
+    if (!(type == 1 ? win_spread_width(dim, ns, elem) : win_interp_width(dim, ns, elem)))
+        return none;
+    if (!win_windows(type, dim, ns, g.nf, w)) return none;
+    if (!win_pays(type, dim, ns, elem, M, ntr, (double)M / w.nkeys))
+        return none;
+    // One wave per range.  Interp: up to 8 rounds of the waves resident on the
+    // device (16 per CU FP32, 8 FP64), no fewer than 128 points each.  Spread: a
+    // range flushes a whole window at its end, so ranges grow to 1536 points before
+    // there are more than half a round of them, and stop at 4 rounds.
+    const int resident = ncu * (elem == 4 ? 16 : 8);
+    if (type == 2)
+        w.ranges = std::max(1, std::min(8 * resident, M / 128));
+    else
+        w.ranges = std::max({1, std::min(resident / 2, M / 128),
+                             std::min(4 * resident, M / 1536)});
+    return w;
+}
+
+int run_win_clear(const SortBufs &sb, long long keys, const Launch &L)
+{
+    const long long b = (keys + 255) / 256;
+    k_fill_int<<<(unsigned)(b < 4096 ? b : 4096), 256, 0, L.stream>>>(keys, 0, sb.wcount);
+    return hipGetLastError() == hipSuccess ? 0 : kErrHip;
+}
+
+template <typename T>
+int run_win_sort(int dim, int M, const SortBufs &sb, const Launch &L)
+{
+    const WinGeom &w = sb.win;
+    const int nparts = (w.nkeys + kScanChunk - 1) / kScanChunk;
+    int2 *part = static_cast<int2 *>(sb.wpart);
+    const SortedPts sp{sb.idx, sb.pos, sb.pos_stride};
+    const int gc = (M + kWinChunk - 1) / kWinChunk;
+    T *x = static_cast<T *>(sb.wx);
+    if (dim == 2)
+        k_win_keys<T, 2, false><<<gc, 512, 0, L.stream>>>(M, sp, w, sb.wcount, nullptr, nullptr,
+                                                          nullptr, nullptr, 0);
+    else
+        k_win_keys<T, 3, false><<<gc, 512, 0, L.stream>>>(M, sp, w, sb.wcount, nullptr, nullptr,
+                                                          nullptr, nullptr, 0);
+    // first points, and with a "subproblem" of 2^30 points the used windows
+    constexpr int kAny = 1 << 30;
+    k_scan_reduce<<<nparts, kScanThreads, 0, L.stream>>>(sb.wcount, w.nkeys, kAny, part);
+    k_scan_parts<<<1, kScanThreads, 0, L.stream>>>(part, nparts,
+                                                   reinterpret_cast<int *>(part + nparts),
+                                                   sb.wused + w.nkeys);
+    k_scan_apply<<<nparts, kScanThreads, 0, L.stream>>>(sb.wcount, w.nkeys, kAny, part, sb.wstart,
+                                                        sb.wused);
+    k_win_ranges<<<w.ranges / 256 + 1, 256, 0, L.stream>>>(M, w.nkeys, w.ranges, sb.wstart,
+                                                           sb.wused, sb.wrange);
+    if (dim == 2)
+        k_win_keys<T, 2, true><<<gc, 512, 0, L.stream>>>(M, sp, w, sb.wcount, sb.wstart, x, sb.wsh,
+                                                         sb.widx, sb.pos_stride);
+    else
+        k_win_keys<T, 3, true><<<gc, 512, 0, L.stream>>>(M, sp, w, sb.wcount, sb.wstart, x, sb.wsh,
+                                                         sb.widx, sb.pos_stride);
+    return hipGetLastError() == hipSuccess ? 0 : kErrHip;
+}
+
+template int run_win_sort<float>(int, int, const SortBufs &, const Launch &);
+template int run_win_sort<double>(int, int, const SortBufs &, const Launch &);
+
+}  // namespace cfa

@@ -1,0 +1,3 @@
+// Window spread kernels for double, 3D.
+#include "win_impl.inl"
+CFA_INSTANTIATE_WIN_SPREAD(double, 3)
