@@ -1741,8 +1741,11 @@ CFA_HD int grid2freq(int l, int ms, int nf)
 CFA_HD int freq2grid(int f, int nf) { return f >= 0 ? f : nf + f; }
 
 // fk[t][k] = fw[t][w(k)] / prod_d fwkerhalf_d[|k_d - ms_d/2|]
-// (Deconvolve_{2,3}d, deconvolve_wrapper.cu:26-66).  One workgroup per output
-// row (fixed k2, k3, t); threads sweep k1 so both reads and writes coalesce.
+// (Deconvolve_{2,3}d, deconvolve_wrapper.cu:26-66).  gridDim.y workgroups per
+// output row (fixed k2, k3, t); threads sweep k1 so both reads and writes
+// coalesce.  Bound by memory once the device is full: few rows are split over
+// workgroups (row_split), one row of 1e5 FP64 modes on a single workgroup took
+// 145 us, on 391 of them 4.7 us.
 template <typename T, int DIM>
 __global__ void __launch_bounds__(256)
 k_deconvolve(int ms, int mt, int mu, int n1, int n2, int n3, const cpx<T> *__restrict__ fw,
@@ -1760,8 +1763,8 @@ k_deconvolve(int ms, int mt, int mu, int n1, int n2, int n3, const cpx<T> *__res
                              (DIM > 1 ? freq2grid(f2, n2) : 0)) *
                                 n1;
         cpx<T> *dst = fk + r * ms;
-        for (int k1 = threadIdx.x; k1 < ms; k1 += blockDim.x) {
-            const int f1 = k1 - ms / 2;
+        for (unsigned k1 = blockIdx.y * 256 + threadIdx.x; k1 < (unsigned)ms; k1 += 256 * gridDim.y) {
+            const int f1 = (int)k1 - ms / 2;
             const T kv = ker1[abs(f1)] * kyz;
             const cpx<T> v = src[freq2grid(f1, n1)];
             cpx<T> o;
@@ -1778,6 +1781,7 @@ k_deconvolve(int ms, int mt, int mu, int n1, int n2, int n3, const cpx<T> *__res
 // the modes are also multiplied by i * wsign * k_wax (k_wax the frequency
 // along axis wax): the type-2 transform of those modes is the derivative of
 // c_j = sum_k f_k e^{i wsign k.x_j} with respect to x_j along that axis.
+// Rows are split over gridDim.y workgroups as in k_deconvolve.
 template <typename T, int DIM>
 __global__ void __launch_bounds__(256)
 k_amplify(int ms, int mt, int mu, int n1, int n2, int n3, cpx<T> *__restrict__ fw,
@@ -1795,7 +1799,8 @@ k_amplify(int ms, int mt, int mu, int n1, int n2, int n3, cpx<T> *__restrict__ f
         zero.x = 0;
         zero.y = 0;
         if (f2 == INT32_MIN || f3 == INT32_MIN) {
-            for (int l1 = threadIdx.x; l1 < n1; l1 += blockDim.x) dst[l1] = zero;
+            for (unsigned l1 = blockIdx.y * 256 + threadIdx.x; l1 < (unsigned)n1; l1 += 256 * gridDim.y)
+                dst[l1] = zero;
             continue;
         }
         const T kyz = (DIM > 1 ? ker2[abs(f2)] : (T)1) * (DIM > 2 ? ker3[abs(f3)] : (T)1);
@@ -1803,8 +1808,8 @@ k_amplify(int ms, int mt, int mu, int n1, int n2, int n3, cpx<T> *__restrict__ f
             fk + t * ntot + ((long long)(f3 + mu / 2) * mt + (f2 + mt / 2)) * (long long)ms;
         // weight i * wsign * k of a fixed row axis (y or z), or per cell (x)
         const T wrow = wax == 1 ? (T)(wsign * f2) : (wax == 2 ? (T)(wsign * f3) : (T)1);
-        for (int l1 = threadIdx.x; l1 < n1; l1 += blockDim.x) {
-            const int f1 = grid2freq(l1, ms, n1);
+        for (unsigned l1 = blockIdx.y * 256 + threadIdx.x; l1 < (unsigned)n1; l1 += 256 * gridDim.y) {
+            const int f1 = grid2freq((int)l1, ms, n1);
             cpx<T> o = zero;
             if (f1 != INT32_MIN) {
                 const T kv = ker1[abs(f1)] * kyz;

@@ -140,13 +140,23 @@ int run_interp(int method, int dim, int ns, int M, const SortBufs &sb, cpx<T> *c
     return interp_dim<T, 3>(method, ns, M, sb, c, fw, g, kp, maxsub, sub_bound, ntr, nftot, L);
 }
 
+// Workgroups for `rows` rows of n cells: one per row where the rows alone give a
+// CU 16 of them (enough waves to cover memory latency), else rows are split, down
+// to one cell per thread.
+static dim3 row_split(long long rows, int n, int ncu)
+{
+    const long long gx = rows < (long long)ncu * 64 ? rows : (long long)ncu * 64;
+    const long long want = ((long long)ncu * 16 + gx - 1) / gx, most = ((long long)n + 255) / 256;
+    return dim3((unsigned)gx, (unsigned)(want < most ? want : most));
+}
+
 template <typename T>
 int run_deconvolve(int dim, const int *ms, const int *nf, const cpx<T> *fw, cpx<T> *fk,
                    const T *const *ker, int ntr, const Launch &L)
 {
     const long long rows = (long long)ms[1] * ms[2] * ntr;
     const long long nftot = (long long)nf[0] * nf[1] * nf[2];
-    const int grid = (int)(rows < (long long)L.ncu * 64 ? rows : (long long)L.ncu * 64);
+    const dim3 grid = row_split(rows, ms[0], L.ncu);
     if (dim == 1)
         k_deconvolve<T, 1><<<grid, 256, 0, L.stream>>>(ms[0], ms[1], ms[2], nf[0], nf[1], nf[2],
                                                        fw, fk, ker[0], ker[1], ker[2], rows,
@@ -168,7 +178,7 @@ int run_amplify(int dim, const int *ms, const int *nf, cpx<T> *fw, const cpx<T> 
 {
     const long long rows = (long long)nf[1] * nf[2] * ntr;
     const long long ntot = (long long)ms[0] * ms[1] * ms[2];
-    const int grid = (int)(rows < (long long)L.ncu * 64 ? rows : (long long)L.ncu * 64);
+    const dim3 grid = row_split(rows, nf[0], L.ncu);
     if (dim == 1)
         k_amplify<T, 1><<<grid, 256, 0, L.stream>>>(ms[0], ms[1], ms[2], nf[0], nf[1], nf[2], fw,
                                                     fk, ker[0], ker[1], ker[2], rows, ntot, wax, wsign);
