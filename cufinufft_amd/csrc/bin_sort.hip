@@ -12,9 +12,11 @@
 // Here the key (the bin, or bin and fine cell for gpu_sort = 2) is sorted
 // in one to three counting passes of at most 10 digit bits each, least
 // significant digit first.  Every pass is a per-tile digit histogram in LDS,
-// one exclusive scan of the (digit, tile) counts over the whole array, and a
-// stable scatter in which each wave ranks its own items among equal digits
-// with ballots (no same-address atomics at any point density).  The payload
+// one exclusive scan of each digit's tile counts (the scatter scans the digit
+// totals itself), and a stable scatter in which each wave ranks its own items
+// among equal digits with ballots (no same-address atomics at any point
+// density).  Where one pass of bin keys does the sort, the digits are the bins,
+// and the scatter also writes the bin tables: 3 launches.  The payload
 // is the point itself -- its coordinates and input index -- so the last pass
 // writes the sorted index and the rescaled positions the execute kernels
 // stream, with no gather through the index afterwards.  The result is the
@@ -92,7 +94,8 @@ __device__ __forceinline__ void load_rec(long long j, const T *__restrict__ x,
 }
 
 // Pass histogram: counts[d * tiles + t] = items of tile t whose digit is d.
-template <typename T, int DIM, bool FINE, bool FIRST>
+// Tiles of 256 R points.
+template <typename T, int DIM, bool FINE, bool FIRST, int R>
 __global__ void __launch_bounds__(256)
 k_sort_hist(int M, const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
             BinGeom g, const int *__restrict__ kin, int shift, int dbits,
@@ -102,10 +105,10 @@ k_sort_hist(int M, const T *__restrict__ x, const T *__restrict__ y, const T *__
     const int nd = 1 << dbits;
     for (int d = threadIdx.x; d < nd; d += 256) h[d] = 0;
     __syncthreads();
-    const long long base = (long long)blockIdx.x * kSortTile;
+    constexpr int kPer = R;
+    const long long base = (long long)blockIdx.x * (256 * R);
     // all of a thread's loads in flight before the first wait, then the keys
     // and their counts
-    constexpr int kPer = kSortTile / 256;
     if constexpr (FIRST) {
         T v[kPer][3];
 #pragma unroll
@@ -137,10 +140,45 @@ k_sort_hist(int M, const T *__restrict__ x, const T *__restrict__ y, const T *__
     for (int d = threadIdx.x; d < nd; d += 256) counts[(long long)d * tiles + blockIdx.x] = h[d];
 }
 
-// Pass scatter.  counts holds the exclusive scan of the histogram, so
-// counts[d * tiles + t] is where tile t's first item of digit d goes.  Wave w
-// of the tile owns items [t * tile + w * 1024, + 1024) in 16 rounds of 64:
-// first it counts its digits; the tile's digit totals are scanned into the
+// One workgroup per digit: exclusive scan of its tile counts in place, and the
+// digit's total.
+static __global__ void __launch_bounds__(kScanThreads)
+k_digit_scan(int tiles, int *__restrict__ counts, int *__restrict__ tot)
+{
+    counts += (long long)blockIdx.x * tiles;
+    int carry = 0;
+    for (int base = 0; base < tiles; base += kScanChunk) {
+        int v[kScanItems], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            const int i = base + threadIdx.x * kScanItems + k;
+            v[k] = i < tiles ? counts[i] : 0;
+            sum += v[k];
+        }
+        int2 ex;
+        const int2 all = block_exscan2(make_int2(sum, 0), ex);
+        int run = carry + ex.x;
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            const int i = base + threadIdx.x * kScanItems + k;
+            if (i < tiles) counts[i] = run;
+            run += v[k];
+        }
+        carry += all.x;
+    }
+    if (threadIdx.x == 0) tot[blockIdx.x] = carry;
+}
+
+// The bin tables a single-pass scatter writes (see run_bin_sort).
+struct BinTables {
+    int nbins, maxsub;
+    int *binsize, *binstart, *substart, *counters, *s2b;  // s2b: may be null
+};
+
+// Pass scatter.  tot holds the items of each digit, and counts[d * tiles + t]
+// how many of them lie in the tiles before t: together where tile t's first
+// item of digit d goes.  Wave w of the tile owns items [t * tile + w * 64 R,
+// + 64 R) in R rounds of 64: first it counts its digits; the tile's digit totals are scanned into the
 // tile-local start of every digit, and each wave's base within a digit
 // follows in wave order; then each round ranks its lanes among equal digits
 // with ballots (the lowest lane of a group advances the base), so equal keys
@@ -149,37 +187,45 @@ k_sort_hist(int M, const T *__restrict__ x, const T *__restrict__ y, const T *__
 // out from there: consecutive threads take consecutive sorted items, whose
 // destinations are consecutive within each digit's run, so the records of a
 // run leave as whole cache lines instead of one line per lane.  LAST writes
-// the sorted key, index and rescaled positions instead of the records.
-template <typename T, int DIM, bool FINE, bool FIRST, bool LAST>
+// the sorted key, index and rescaled positions instead of the records; BINS (one
+// pass, digit = bin) no key but the bin tables.
+//
+// Latency bounds it below a few 1e5 points: a tile's R rounds follow each other.
+// Tiles of 1024 points take 8 us for 4001 2D points (4096: 16 us) and 15 us for
+// 1e6 1D points (21 us); with the 3 launches instead of 11 the sort of 4001
+// points takes 15 us instead of 41 us.
+template <typename T, int DIM, bool FINE, bool FIRST, bool LAST, bool BINS, int R>
 __global__ void __launch_bounds__(256)
 k_sort_scatter(int M, const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
                BinGeom g, const int *__restrict__ kin, const SortRec<T, DIM> *__restrict__ rin,
                int shift, int dbits, const int *__restrict__ counts, int tiles,
                int *__restrict__ kout, SortRec<T, DIM> *__restrict__ rout,
-               int *__restrict__ idx, double *__restrict__ pos, long long stride)
+               int *__restrict__ idx, double *__restrict__ pos, long long stride,
+               const int *__restrict__ dtot, BinTables bt)
 {
+    constexpr int kRounds = R, kTile = 256 * R;
     constexpr int kMaxDigits = 1 << kMaxDigitBits;
     constexpr int kPer = kMaxDigits / 256;  // digits per thread in the tile scan
     __shared__ int wb[kSortWaves][kMaxDigits];
     __shared__ int dl[kMaxDigits];  // tile-local start of each digit's items
     __shared__ int gd[kMaxDigits];  // global start of them
-    __shared__ int sk[kSortTile];   // the tile's keys in sorted order
-    __shared__ int sj[kSortTile];   // and their input positions
+    __shared__ int sk[kTile];   // the tile's keys in sorted order
+    __shared__ int sj[kTile];   // and their input positions
     const int nd = 1 << dbits;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int d = threadIdx.x; d < nd; d += 256)
 #pragma unroll
         for (int q = 0; q < kSortWaves; ++q) wb[q][d] = 0;
     __syncthreads();
-    const long long tbase = (long long)blockIdx.x * kSortTile;
-    const long long wbase = tbase + w * (kSortRounds * 64);
-    int keys[kSortRounds];  // this lane's keys, kept for the ranking rounds
+    const long long tbase = (long long)blockIdx.x * kTile;
+    const long long wbase = tbase + w * (kRounds * 64);
+    int keys[kRounds];  // this lane's keys, kept for the ranking rounds
     // all of the lane's loads in flight before the first wait, then the keys
     // and their counts
     if constexpr (FIRST) {
-        T v[kSortRounds][3];
+        T v[kRounds][3];
 #pragma unroll
-        for (int r = 0; r < kSortRounds; ++r) {
+        for (int r = 0; r < kRounds; ++r) {
             const long long j = wbase + r * 64 + lane;
             v[r][0] = v[r][1] = v[r][2] = T(0);
             if (j < M) {
@@ -189,26 +235,28 @@ k_sort_scatter(int M, const T *__restrict__ x, const T *__restrict__ y, const T 
             }
         }
 #pragma unroll
-        for (int r = 0; r < kSortRounds; ++r) keys[r] = sort_key<T, DIM, FINE>(v[r], g);
+        for (int r = 0; r < kRounds; ++r) keys[r] = sort_key<T, DIM, FINE>(v[r], g);
     } else {
 #pragma unroll
-        for (int r = 0; r < kSortRounds; ++r) {
+        for (int r = 0; r < kRounds; ++r) {
             const long long j = wbase + r * 64 + lane;
             keys[r] = j < M ? kin[j] : 0;
         }
     }
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
         if (wbase + r * 64 + lane < M)
             atomicAdd(&wb[w][(keys[r] >> shift) & (nd - 1)], 1);
         else
             keys[r] = 0;  // items past M are never ranked or written
     }
     __syncthreads();
-    // digit totals of the tile (thread t owns digits kPer t .. kPer t + kPer-1),
-    // their exclusive scan, and each wave's tile-local base per digit
+    // digit totals of the tile (thread t owns digits kPer t .. kPer t + kPer-1)
+    // and of the whole array, their exclusive scans, and each wave's tile-local
+    // base per digit
     int tot[kPer];
     int sum = 0;
+    int2 all[kPer], asum = make_int2(0, 0);  // items, subproblems (BINS)
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         const int d = threadIdx.x * kPer + k;
@@ -217,16 +265,20 @@ k_sort_scatter(int M, const T *__restrict__ x, const T *__restrict__ y, const T 
 #pragma unroll
             for (int q = 0; q < kSortWaves; ++q) tot[k] += wb[q][d];
         sum += tot[k];
+        all[k] = d < nd ? load_pair(dtot, d, nd, BINS ? bt.maxsub : 1) : make_int2(0, 0);
+        asum = add2(asum, all[k]);
     }
     int2 ex;
     block_exscan2(make_int2(sum, 0), ex);
     int run = ex.x;
+    int2 arun;
+    const int2 atot = block_exscan2(asum, arun);
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         const int d = threadIdx.x * kPer + k;
         if (d < nd) {
             dl[d] = run;
-            gd[d] = counts[(long long)d * tiles + blockIdx.x];
+            gd[d] = arun.x + counts[(long long)d * tiles + blockIdx.x];
             int b = run;
 #pragma unroll
             for (int q = 0; q < kSortWaves; ++q) {
@@ -236,11 +288,26 @@ k_sort_scatter(int M, const T *__restrict__ x, const T *__restrict__ y, const T 
             }
             run += tot[k];
         }
+        if (BINS && d < bt.nbins) {
+            if (blockIdx.x == 0) {
+                bt.binsize[d] = all[k].x;
+                bt.binstart[d] = arun.x;
+                bt.substart[d] = arun.y;
+            }
+            if (bt.s2b && d % gridDim.x == blockIdx.x)
+                for (int s = 0; s < all[k].y; ++s) bt.s2b[arun.y + s] = d;
+        }
+        arun = add2(arun, all[k]);
+    }
+    if (BINS && blockIdx.x == 0 && threadIdx.x == 0) {
+        bt.substart[bt.nbins] = atot.y;
+        bt.counters[0] = atot.x;
+        bt.counters[1] = atot.y;
     }
     __syncthreads();
     const unsigned long long lt = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
         const long long j = wbase + r * 64 + lane;
         const bool act = j < M;
         const int d = act ? (keys[r] >> shift) & (nd - 1) : 0;
@@ -263,9 +330,9 @@ k_sort_scatter(int M, const T *__restrict__ x, const T *__restrict__ y, const T 
     // write-out in batches of kBatch items per thread: all of a batch's
     // record loads are issued before the first store, so their latencies
     // overlap instead of adding up item by item
-    const int nt = (int)(M - tbase < kSortTile ? M - tbase : kSortTile);
-    constexpr int kBatch = 8;
-    for (int b0 = 0; b0 < kSortTile; b0 += 256 * kBatch) {
+    const int nt = (int)(M - tbase < kTile ? M - tbase : kTile);
+    constexpr int kBatch = R < 8 ? R : 8;
+    for (int b0 = 0; b0 < kTile; b0 += 256 * kBatch) {
         SortRec<T, DIM> rec[kBatch];
         int key[kBatch];
 #pragma unroll
@@ -283,7 +350,7 @@ k_sort_scatter(int M, const T *__restrict__ x, const T *__restrict__ y, const T 
             if (lp < nt) {
                 const int d = (key[k] >> shift) & (nd - 1);
                 const int dst = gd[d] + (lp - dl[d]);
-                kout[dst] = key[k];
+                if (!BINS) kout[dst] = key[k];
                 if constexpr (LAST) {
                     idx[dst] = rec[k].i;
 #pragma unroll
@@ -341,25 +408,43 @@ k_run_sizes(int M, int vol, const int *__restrict__ skey, int *__restrict__ bins
 
 namespace {
 
-// Exclusive scan of n ints in place (the int2 scan kernels with the second
-// component unused).
-void scan_inplace(int *a, long long n, int2 *part, const Launch &L)
+// One pass over all key bits.  BINS: the keys are bins, whose tables bt it writes.
+// R = 4 tiles where 4096-point ones (R = 16) would not give every CU one, as far
+// as their counts fit the second key buffer, which no single pass uses.
+template <typename T, int DIM, bool FINE, bool BINS, int R>
+int sort_single(int M, const T *x, const T *y, const T *z, const BinGeom &g, int bits,
+                const BinTables &bt, SortBufs &sb, const Launch &L)
 {
-    const long long nparts = (n + kScanChunk - 1) / kScanChunk;
-    k_scan_reduce<<<(unsigned)nparts, kScanThreads, 0, L.stream>>>(a, n, 1, part);
-    k_scan_parts<<<1, kScanThreads, 0, L.stream>>>(part, (int)nparts, nullptr, nullptr);
-    k_scan_apply<<<(unsigned)nparts, kScanThreads, 0, L.stream>>>(a, n, 1, part, a, nullptr);
+    const int tiles = (int)(((long long)M + 256 * R - 1) / (256 * R));
+    int *counts = R == kSortRounds ? sb.sort_counts : sb.skey_out;
+    k_sort_hist<T, DIM, FINE, true, R><<<tiles, 256, 0, L.stream>>>(M, x, y, z, g, nullptr, 0,
+                                                                    bits, counts, tiles);
+    k_digit_scan<<<1 << bits, kScanThreads, 0, L.stream>>>(tiles, counts, sb.sort_tot);
+    k_sort_scatter<T, DIM, FINE, true, true, BINS, R><<<tiles, 256, 0, L.stream>>>(
+        M, x, y, z, g, nullptr, nullptr, 0, bits, counts, tiles, sb.skey, nullptr, sb.idx, sb.pos,
+        sb.pos_stride, sb.sort_tot, bt);
+    return ok_or_err();
+}
+template <typename T, int DIM, bool FINE, bool BINS>
+int sort_single(int M, const T *x, const T *y, const T *z, const BinGeom &g, int bits,
+                const BinTables &bt, SortBufs &sb, const Launch &L)
+{
+    const bool small = (long long)M <= (long long)L.ncu * kSortTile &&
+                       ((((long long)M + 1023) / 1024) << bits) <= M;
+    return small ? sort_single<T, DIM, FINE, BINS, 4>(M, x, y, z, g, bits, bt, sb, L)
+                 : sort_single<T, DIM, FINE, BINS, kSortRounds>(M, x, y, z, g, bits, bt, sb, L);
 }
 
 template <typename T, int DIM, bool FINE>
 int sort_passes(int M, const T *x, const T *y, const T *z, const BinGeom &g,
                 const BinSortShape &sh, SortBufs &sb, const Launch &L)
 {
+    if (sh.passes == 1)
+        return sort_single<T, DIM, FINE, false>(M, x, y, z, g, sh.bits, BinTables{}, sb, L);
     using Rec = SortRec<T, DIM>;
     Rec *rec[2] = {reinterpret_cast<Rec *>(sb.rec[0]), reinterpret_cast<Rec *>(sb.rec[1])};
     int *keys[2] = {sb.skey, sb.skey_out};
     const long long st = sb.pos_stride;
-    int2 *part = static_cast<int2 *>(sb.sort_part);
     const int tiles = sh.tiles;
     for (int p = 0; p < sh.passes; ++p) {
         const int shift = p * sh.digit_bits;
@@ -367,19 +452,18 @@ int sort_passes(int M, const T *x, const T *y, const T *z, const BinGeom &g,
         const int in = (p + 1) & 1, out = p & 1;  // pass p writes buffer p % 2
         const bool first = p == 0, last = p + 1 == sh.passes;
         if (first)
-            k_sort_hist<T, DIM, FINE, true><<<tiles, 256, 0, L.stream>>>(
+            k_sort_hist<T, DIM, FINE, true, kSortRounds><<<tiles, 256, 0, L.stream>>>(
                 M, x, y, z, g, nullptr, shift, dbits, sb.sort_counts, tiles);
         else
-            k_sort_hist<T, DIM, FINE, false><<<tiles, 256, 0, L.stream>>>(
+            k_sort_hist<T, DIM, FINE, false, kSortRounds><<<tiles, 256, 0, L.stream>>>(
                 M, x, y, z, g, keys[in], shift, dbits, sb.sort_counts, tiles);
-        scan_inplace(sb.sort_counts, (long long)tiles << dbits, part, L);
+        k_digit_scan<<<1 << dbits, kScanThreads, 0, L.stream>>>(tiles, sb.sort_counts,
+                                                                sb.sort_tot);
 #define CFA_SCATTER(F, LST)                                                                   \
-    k_sort_scatter<T, DIM, FINE, F, LST><<<tiles, 256, 0, L.stream>>>(                        \
+    k_sort_scatter<T, DIM, FINE, F, LST, false, kSortRounds><<<tiles, 256, 0, L.stream>>>(    \
         M, x, y, z, g, keys[in], rec[in], shift, dbits, sb.sort_counts, tiles, keys[out],     \
-        rec[out], sb.idx, sb.pos, st)
-        if (first && last)
-            CFA_SCATTER(true, true);
-        else if (first)
+        rec[out], sb.idx, sb.pos, st, sb.sort_tot, BinTables{})
+        if (first)
             CFA_SCATTER(true, false);
         else if (last)
             CFA_SCATTER(false, true);
@@ -398,6 +482,16 @@ int run_bin_sort(int dim, const BinGeom &g, long long nbins, int M, const T *x, 
                  const Launch &L)
 {
     const int vol = fine ? g.bs[0] * g.bs[1] * g.bs[2] : 1;
+    if (M > 0 && !fine) {
+        const BinSortShape sh = bin_sort_shape(M, nbins);
+        if (sh.passes == 1) {
+            const BinTables bt{(int)nbins,  maxsub,      sb.binsize, sb.binstart,
+                               sb.substart, sb.counters, need_subprob ? sb.s2b : nullptr};
+            if (dim == 1) return sort_single<T, 1, false, true>(M, x, y, z, g, sh.bits, bt, sb, L);
+            if (dim == 2) return sort_single<T, 2, false, true>(M, x, y, z, g, sh.bits, bt, sb, L);
+            return sort_single<T, 3, false, true>(M, x, y, z, g, sh.bits, bt, sb, L);
+        }
+    }
     k_fill_int<<<grid_pts(nbins, L.ncu), 256, 0, L.stream>>>(nbins, 0, sb.binsize);
     int e = 0;
     if (M > 0) {

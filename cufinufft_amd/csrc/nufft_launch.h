@@ -55,7 +55,7 @@ struct SortBufs {
     int *skey_out = nullptr;    // [M] sort keys, pass ping-pong buffer 1
     void *rec[2] = {nullptr, nullptr};  // [M] point records between sort passes
     int *sort_counts = nullptr; // (digit, tile) counts of one sort pass
-    void *sort_part = nullptr;  // int2 partial sums of their scan
+    int *sort_tot = nullptr;    // [1 << kMaxDigitBits] items of each digit
     int *idx = nullptr;         // [M] caller index of each sorted point
     double *pos = nullptr;      // [dim][pos_stride] sorted rescaled positions
     long long pos_stride = 0;   // capacity in points of each pos plane

@@ -534,8 +534,7 @@ struct Plan {
             r = nullptr;
         }
         dfree(sb.sort_counts);
-        if (sb.sort_part) hipFree(sb.sort_part);
-        sb.sort_part = nullptr;
+        dfree(sb.sort_tot);
         dfree(sb.idx);
         dfree(sb.pos);
         dfree(sb.counters);
@@ -972,7 +971,7 @@ int Plan<T>::makeplan(int type_, int dim_, const int *nmodes, int iflag_, int nt
     }
     if (dmalloc(&sb.binsize, nbins) || dmalloc(&sb.binstart, nbins) ||
         dmalloc(&sb.substart, nbins + 1) || dmalloc(&sb.counters, 2) ||
-        dmalloc(&sb.jobq, kJobqWords) ||
+        dmalloc(&sb.jobq, kJobqWords) || dmalloc(&sb.sort_tot, 1 << kMaxDigitBits) ||
         hipMemset(sb.jobq, 0, kJobqWords * sizeof(unsigned long long)) != hipSuccess)
         return kErrHip;
     const long long nparts = (nbins + kScanChunk - 1) / kScanChunk;
@@ -1119,20 +1118,15 @@ int Plan<T>::setpts(int M_, const T *x, const T *y, const T *z)
         sb.pos_stride = M;
     }
     if (method != 4 && !(method == 1 && !opts.gpu_sort) && M > 0) {
-        // counting-sort scratch: (digit, tile) counts and their scan
-        // partials, and the point records between passes (none for one pass)
+        // counting-sort scratch: (digit, tile) counts, and the point records
+        // between passes (none for one pass)
         const long long nkeys =
             opts.gpu_sort == 2 ? nbins * (long long)geom.bs[0] * geom.bs[1] * geom.bs[2] : nbins;
         const BinSortShape sh = bin_sort_shape(M, nkeys);
         if (sh.counts > cap_counts) {
             dfree(sb.sort_counts);
-            if (sb.sort_part) hipFree(sb.sort_part);
-            sb.sort_part = nullptr;
             cap_counts = -1;
-            const long long parts = (sh.counts + kScanChunk - 1) / kScanChunk;
-            if (dmalloc(&sb.sort_counts, (size_t)sh.counts) ||
-                hipMalloc(&sb.sort_part, sizeof(int2) * (size_t)parts) != hipSuccess)
-                return kErrHip;
+            if (dmalloc(&sb.sort_counts, (size_t)sh.counts)) return kErrHip;
             cap_counts = sh.counts;
         }
         const size_t rb = bin_sort_rec_bytes(dim, sizeof(T));
@@ -1180,7 +1174,7 @@ int Plan<T>::setpts(int M_, const T *x, const T *y, const T *z)
 
 // setpts without allocation (cufinufftf_setpts_noalloc): the same bin sort,
 // with its transient buffers (the key ping-pong pair, the point records
-// between passes, the per-pass (digit, tile) counts and their scan partials)
+// between passes, the per-pass (digit, tile) counts)
 // carved from the caller-supplied device scratch instead of the plan's own.
 // The plan's lasting point arrays (sorted index, positions, subproblem map)
 // must already hold M points: an earlier setpts of at least M points sized
@@ -1219,7 +1213,7 @@ int Plan<T>::setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned
         s2.rec[0] = sh.passes > 1 ? take(rb * (size_t)M_) : nullptr;
         s2.rec[1] = sh.passes > 2 ? take(rb * (size_t)M_) : nullptr;
         s2.sort_counts = reinterpret_cast<int *>(take(sizeof(int) * (size_t)sh.counts));
-        s2.sort_part = take(sizeof(int2) * (size_t)parts);
+        take(sizeof(int2) * (size_t)parts);  // unused: keeps the limit on M where it was
         if (off > scr_bytes) return kErrNoAlloc;
     }
     DeviceGuard dg(opts.gpu_device_id);

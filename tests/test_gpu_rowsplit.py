@@ -6,7 +6,7 @@ output."""
 import numpy as np
 import pytest
 
-from . import gpu_util as G
+from tests import gpu_util as G
 
 pytestmark = pytest.mark.gpu
 
