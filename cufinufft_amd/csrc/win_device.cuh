@@ -19,8 +19,8 @@
 // clock and CU for 32-bit, 64-bit integer and FP64 LDS adds), the per-point
 // interp one LDS or L1 read and two FMAs per tap.
 // Spread or interp alone, per-point -> window kernel: 3D FP32 type 1, ns 6, 1e8
-// points on 512^3: 20.7 -> 7.9 ms; 3D FP64 type 2, ns 10, 1e7: 17.7 -> 3.4 ms;
-// 2D FP64 type 2: 0.90 -> 0.39 ms (the rule of win_sort.hip has both sides at
+// points on 512^3: 20.7 -> 6.9 ms; 3D FP64 type 2, ns 10, 1e7: 17.7 -> 3.3 ms;
+// 2D FP64 type 2: 0.90 -> 0.35 ms (the rule of win_sort.hip has both sides at
 // the edges of its range).
 #pragma once
 #include <utility>
@@ -74,6 +74,18 @@ __device__ __forceinline__ double dpp(double old, double v)
     const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf,
                                                BANKS, false);
     return __hiloint2double(hi, lo);
+}
+// Broadcast of lane N of each row.
+template <int N>
+__device__ __forceinline__ float row_bcast(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ double row_bcast(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + N, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + N, 0xf, 0xf, true));
 }
 constexpr int kDppBcast = 0x150, kDppRor = 0x120, kDppShl = 0x100, kDppShr = 0x110;
 
@@ -139,27 +151,27 @@ __device__ __forceinline__ double win_exp(double x)
 }
 
 // Kernel value at offset x from the point, over its peak: phi(x) / e^beta; the
-// callers put e^(DIM beta) back in FP64.  Outside the support, and for ok =
-// false, the exponent is replaced by one that underflows to 0, so the code has
-// no branch: many evaluations overlap.
+// callers put e^(DIM beta) back in FP64.  Outside the support the exponent is
+// replaced by one that underflows to 0, so the code has no branch: many
+// evaluations overlap.
 //
 // FP32 forms the exponent beta (sqrt(1 - t) - 1), t = c x^2, as -beta t /
 // (1 + sqrt(1 - t)): its rounding is then relative to the exponent, which is
 // small where the kernel is large, and the hardware square root and reciprocal
 // (1 ulp) do.  The difference sqrt(..) - 1 itself carries half an ulp of 1, times
 // beta (14 - 20) a relative error of ~3e-7 in every weight.
-__device__ __forceinline__ float win_phi(float x, const KerParams<float> &k, bool ok = true)
+__device__ __forceinline__ float win_phi(float x, const KerParams<float> &k)
 {
     const float t = k.c * x * x;
     const float s = __builtin_amdgcn_sqrtf(fmaxf(1.0f - t, 0.0f));
     const float w = t * __builtin_amdgcn_rcpf(1.0f + s);
     const float e = fmaf(-k.bl2e, w, -k.bl2e_lo * w);
-    return __builtin_amdgcn_exp2f(((fabsf(x) < k.hw) & ok) ? e : -1000.0f);
+    return __builtin_amdgcn_exp2f(fabsf(x) < k.hw ? e : -1000.0f);
 }
-__device__ __forceinline__ double win_phi(double x, const KerParams<double> &k, bool ok = true)
+__device__ __forceinline__ double win_phi(double x, const KerParams<double> &k)
 {
     const double v = win_exp(k.beta * (win_sqrt(fmax(1.0 - k.c * x * x, 0x1p-60)) - 1.0));
-    return ((fabs(x) < k.hw) & ok) ? v : 0.0;
+    return fabs(x) < k.hw ? v : 0.0;
 }
 
 // Place of a point (position v, in [-1, nf + 1]) along one axis: its first tap
@@ -265,11 +277,38 @@ struct WinKeys {
     }
 };
 
-// A staged point in LDS.
-template <typename T>
-struct alignas(4 * sizeof(T)) WinRec {
-    T x[3];
-    unsigned sh;  // first tap inside its window, a byte per axis
+// The weights of a point in LDS: its NS weights along x, a zero, those along y, a
+// zero, and (3D) those along z.  A wave's lanes are points when the weights are
+// evaluated, so each is evaluated once, and window cells when they are used: a
+// cell reads the weight of tap (cell - first tap), or the zero behind the taps.
+// The pitch is odd: the lanes' rows start in different banks.
+template <typename T, int DIM, int NS>
+struct WinRow {
+    static constexpr int Y = NS + 1, Z = 2 * NS + 2;
+    static constexpr int pitch = (DIM == 3 ? 3 * NS + 2 : 2 * NS + 2) | 1;
+    // Index of tap i of an axis, of its zero where i is none of the NS taps.
+    __device__ static __forceinline__ int tap(int i) { return (int)min((unsigned)i, (unsigned)NS); }
+    __device__ static __forceinline__ void clear(T *rows, int n, int lane)
+    {
+        for (int k = lane; k < 2 * n; k += 64) rows[(k >> 1) * pitch + (k & 1 ? Y : 0) + NS] = T(0);
+    }
+    // Weights of an axis at f (see win_place), and the half h of the z weights.
+    __device__ static __forceinline__ void axis(T *w, T f, const KerParams<T> &kp)
+    {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) w[i] = win_phi(f + ((T)i - T(0.5) * NS), kp);
+    }
+    __device__ static __forceinline__ void half(T *w, int h, T f, const KerParams<T> &kp)
+    {
+        constexpr int N = (NS + 1) / 2;
+        w += h * N;
+        f += (T)(h * N) - T(0.5) * NS;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const T v = win_phi(f + (T)i, kp);
+            if (i + 1 < N || NS % 2 == 0 || h == 0) w[i] = v;
+        }
+    }
 };
 
 // ---------------------------------------------------------------------------
@@ -282,15 +321,18 @@ struct alignas(4 * sizeof(T)) WinRec {
 // common scale and no barrier is needed.  In 2D a window is one such plane,
 // and NT transforms share the weights.
 //
-// Bounds per point (rate of a CU): 4 ns (FP32) or 8 ns clocks of the matrix
-// cores in 3D, about 20 VALU instructions for the weights, and the atomics, at
-// 3.0e11 (FP32) or 1.75e11 (FP64) lanes per second on the whole device.
+// Bounds per 4 points and SIMD: 64 ns (FP32) or 128 ns clocks of the matrix cores
+// in 3D, about 110 for the operands and 120 for the weights (which took 240 when
+// each lane evaluated those of its own cell, zeros included: ns 6, 1e8 points on
+// 512^3, 7.87 -> 6.85 ms), and the atomics, 1.9e10 64-byte pieces a second on the
+// whole device (ns 7, 2e7 points on 384^3, 2.28 -> 1.93 ms by place()'s order).
 template <typename T, int DIM, int NS, int NT>
 struct WinSpread {
     using Acc = typename Mfma<T>::Acc;
     static constexpr int RB = DIM == 3 ? NS : 1;
+    static constexpr int kBlock = 32;  // points staged at a time
     Acc ar[NT][RB], ai[NT][RB];
-    unsigned row[4], col[2];  // see place()
+    unsigned row[4], col[2], src[2];  // see place()
 
     __device__ __forceinline__ void clear()
     {
@@ -300,48 +342,58 @@ struct WinSpread {
             for (int m = 0; m < RB; ++m) ar[t][m] = ai[t][m] = Acc{0, 0, 0, 0};
     }
     // The window's place (kx, ky): where in a plane the components go that
-    // flush() hands this lane.
+    // flush() hands this lane (row, col), and their index in a row (src).  Of a
+    // row's 32 components lane i takes two, 16 apart, so that a 16-lane group
+    // covers whole 64-byte pieces of memory but for the row's two ends: 3 pieces a
+    // row in FP32 instead of 4, which is what the memory counts.  Quarter q takes
+    // rows q + 4 r: grid rows have an even length, so 4 of them shift a row by whole
+    // pieces.
     __device__ __forceinline__ void place(int kx, int ky, const BinGeom &g)
     {
         constexpr int S = 17 - NS, F = (NS + 1) / 2 + 1;
         const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            row[r] = 2u * (unsigned)(win_wrap(ky * S - F + mfma_row<T>(q, r), g.nf[1]) * g.nf[0]);
+            row[r] = 2u * (unsigned)(win_wrap(ky * S - F + q + 4 * r, g.nf[1]) * g.nf[0]);
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-            col[b] = 2u * (unsigned)win_wrap(kx * S - F + 8 * b + (i16 >> 1), g.nf[0]) + (i16 & 1);
+        for (int b = 0; b < 2; ++b) {
+            constexpr int cells = 32 / sizeof(T);  // cells of 64 bytes
+            const int at = kx * S - F + (ky * S - F + q) * g.nf[0];
+            src[b] = (unsigned)(16 * b + i16 - 2 * (at & (cells - 1))) & 31;
+            col[b] = 2u * (unsigned)win_wrap(kx * S - F + (int)(src[b] >> 1), g.nf[0]) + (src[b] & 1);
+        }
     }
-    // Points s .. e - 1 of the staged batch (of one window); zslot: slot of
-    // their first plane.
-    __device__ __forceinline__ void accumulate(int s, int e, int zslot, const WinRec<T> *rec,
-                                               const cpx<T> *cs, const KerParams<T> &kp)
+    // Points s .. e - 1 of the staged block (of one window); zslot: slot of their
+    // first plane.
+    __device__ __forceinline__ void accumulate(int s, int e, int zslot, const T *rows,
+                                               const unsigned *sh, const cpx<T> *cs)
     {
+        using Row = WinRow<T, DIM, NS>;
         const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
-        // lane i of a row evaluates the x and y weights of cell i and the z
-        // weight of slot i
-        const T hw = T(0.5) * NS, f = (T)i16 - hw;
-        const int zt = i16 - zslot;
-        const T fz = (T)(zt < 0 ? zt + NS : zt) - hw;
-        for (int b = s; b < e; b += 4) {
-            // quarter q of the wave holds point b + q
-            const bool ok = b + q < e;
+        // lane i of a row takes the x and y weights of cell i and the z weight
+        // of slot i (any weight for i >= ns)
+        const int zt = i16 - zslot, z = Row::Z + min(zt < 0 ? zt + NS : zt, NS - 1);
+        // quarter q of the wave holds point b + q; groups of 4 start at multiples
+        // of 4 of the block, so only a window's first and last are not full
+        for (int b = s & ~3; b < e; b += 4) {
+            const bool ok = b + q >= s && b + q < e;
             const int p = ok ? b + q : s;
-            const WinRec<T> r = rec[p];
-            const T kx = win_phi(r.x[0] + (f - (T)(r.sh & 255)), kp, ok);
-            const T ky = win_phi(r.x[1] + (f - (T)(r.sh >> 8 & 255)), kp);
+            const T *row = rows + __umul24(p, Row::pitch);
+            const unsigned u = sh[p];
+            const T kx = row[ok ? Row::tap(i16 - (int)(u & 255)) : NS];
+            const T ky = row[Row::Y + Row::tap(i16 - (int)(u >> 8 & 255))];
             T kz = T(0);
-            if (DIM == 3) kz = win_phi(r.x[2] + fz, kp);
+            if (DIM == 3) kz = row[z];
             T br[NT], bi[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const cpx<T> v = cs[64 * t + p];
+                const cpx<T> v = cs[kBlock * t + p];
                 br[t] = v.x * kx;
                 bi[t] = v.y * kx;
             }
             static_for<RB>([&](auto mc) {
                 constexpr int m = decltype(mc)::value;
-                const T a = DIM == 3 ? ky * dpp<kDppBcast + m, 0xf>(kz, kz) : ky;
+                const T a = DIM == 3 ? ky * row_bcast<m>(kz) : ky;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     ar[t][m] = Mfma<T>::mac(a, br[t], ar[t][m]);
@@ -360,7 +412,8 @@ struct WinSpread {
     __device__ __forceinline__ void flush(T *plane, long long tstride, int nt, cpx<T> *sc)
     {
         const int lane = threadIdx.x & 63;
-        const T *src = reinterpret_cast<const T *>(sc) + (lane & 48) * 2 + (lane & 15);
+        // row q + 4 r: register r of quarter q in FP64, register q of quarter r in FP32
+        const T *from = reinterpret_cast<const T *>(sc) + (lane >> 4) * (sizeof(T) == 4 ? 128 : 32);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             if (NT == 1 || t < nt) {
@@ -378,7 +431,7 @@ struct WinSpread {
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
-                        const T v = src[128 * r + 16 * b];
+                        const T v = from[(sizeof(T) == 4 ? 32 : 128) * r + src[b]];
                         if (v != T(0)) gadd(p + (row[r] + col[b]), v);
                     }
             }
@@ -393,12 +446,17 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
              WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
 {
     constexpr int F = (NS + 1) / 2 + 1;
-    __shared__ WinRec<T> srec[256];
-    __shared__ cpx<T> scs[256 * NT], ssc[1024];
-    const int lane = threadIdx.x & 63;
+    using Acc = WinSpread<T, DIM, NS, NT>;
+    using Row = WinRow<T, DIM, NS>;
+    constexpr int B = Acc::kBlock;
+    __shared__ T srow[4 * B * Row::pitch];
+    __shared__ unsigned ssh[4 * B];
+    __shared__ cpx<T> scs[4 * B * NT], ssc[1024];
+    const int lane = threadIdx.x & 63, h = lane >> 5, pl = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    WinRec<T> *rec = srec + wave * 64;
-    cpx<T> *cs = scs + wave * 64 * NT, *sc = ssc + wave * 256;
+    T *rows = srow + wave * B * Row::pitch;
+    unsigned *sh = ssh + wave * B;
+    cpx<T> *cs = scs + wave * B * NT, *sc = ssc + wave * 256;
     const T *x1 = static_cast<const T *>(wp.x);
     const JobRange jr = xcd_jobs(gridDim.x);  // one range per wave, contiguous per XCD
     const int rng = (int)jr.begin * 4 + wave;
@@ -410,33 +468,39 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
     c += (long long)t0 * M;
     T *ft = reinterpret_cast<T *>(fw + (long long)t0 * nftot);
     const double back = exp((double)DIM * (double)kp.beta);
-    WinSpread<T, DIM, NS, NT> acc;
+    Acc acc;
     acc.clear();
+    Row::clear(rows, B, lane);
     WinKeys keys;
     keys.load(wp, wg.nkeys, win_key_of(wp.start, wg.nkeys, p));
-    // batches of 64 points, one per lane: the next batch's strengths and the
-    // records of the one after are in flight while one is worked on
-    T xa[DIM], xb[DIM];
+    // blocks of 32 points: lane l has point l % 32 and, half h of the wave, axis h
+    // (and a half of the z weights), and the transforms t = h mod 2.  The next
+    // block's strengths and the records of the one after are in flight while one
+    // is worked on
+    constexpr int NC = (NT + 1) / 2;
+    T xa, za = T(0), xb, zb = T(0);
     unsigned sa, sb;
     int ib;
-    cpx<T> ca[NT];
-    auto load = [&](int i, T *x, unsigned &s, int &id) {
+    cpx<T> ca[NC];
+    const T *xh = x1 + h * wp.stride;
+    auto load = [&](int i, T &x, T &z, unsigned &s, int &id) {
         const int k = min(i, pe - 1);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) x[d] = x1[d * wp.stride + k];
+        x = xh[k];
+        if (DIM == 3) z = x1[2 * wp.stride + k];
         s = wp.sh[k];
         id = wp.idx[k];
     };
     auto gather = [&](int id) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            ca[t].x = ca[t].y = T(0);
-            if (NT == 1 || t < nt) ca[t] = c[(long long)t * M + id];
+        for (int j = 0; j < NC; ++j) {
+            const int t = 2 * j + h;
+            ca[j].x = ca[j].y = T(0);
+            if (t < nt) ca[j] = c[(long long)t * M + id];
         }
     };
-    load(p + lane, xa, sa, ib);
+    load(p + pl, xa, za, sa, ib);
     gather(ib);
-    load(p + 64 + lane, xb, sb, ib);
+    load(p + B + pl, xb, zb, sb, ib);
     int b0 = p;
     bool staged = false;
     int strip = -1, z = 0;  // window held (3D: its first plane's place too)
@@ -456,7 +520,7 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
         for (int k = z; k < z + nf; ++k) {
             T *plane = ft + (DIM == 3 ? win_wrap(k - F, g.nf[2]) * pstride : 0);
             const int m = DIM == 3 ? k % NS : 0;
-            static_for<WinSpread<T, DIM, NS, NT>::RB>([&](auto mc) {
+            static_for<Acc::RB>([&](auto mc) {
                 if (m == decltype(mc)::value)
                     acc.template flush<decltype(mc)::value>(plane, 2 * nftot, nt, sc);
             });
@@ -466,30 +530,29 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
         strip = st;
         z = zk;
         while (p < ke) {
-            if (!staged || p >= b0 + 64) {
-                if (staged) b0 += 64;
+            if (!staged || p >= b0 + B) {
+                if (staged) b0 += B;
                 staged = true;
                 __builtin_amdgcn_wave_barrier();
-                WinRec<T> r;
+                T *row = rows + pl * Row::pitch;
+                Row::axis(row + h * Row::Y, xa, kp);
+                if (DIM == 3) Row::half(row + Row::Z, h, za, kp);
+                sh[pl] = sa;
 #pragma unroll
-                for (int d = 0; d < DIM; ++d) r.x[d] = xa[d];
-                r.sh = sa;
-                rec[lane] = r;
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    ca[t].x = (T)((double)ca[t].x * back);
-                    ca[t].y = (T)((double)ca[t].y * back);
-                    cs[64 * t + lane] = ca[t];
+                for (int j = 0; j < NC; ++j) {
+                    ca[j].x = (T)((double)ca[j].x * back);
+                    ca[j].y = (T)((double)ca[j].y * back);
+                    if (2 * j + h < NT) cs[B * (2 * j + h) + pl] = ca[j];
                 }
                 gather(ib);
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) xa[d] = xb[d];
+                xa = xb;
+                za = zb;
                 sa = sb;
-                load(b0 + 128 + lane, xb, sb, ib);
+                load(b0 + 2 * B + pl, xb, zb, sb, ib);
                 __builtin_amdgcn_wave_barrier();
             }
-            const int e = min(ke, b0 + 64);
-            acc.accumulate(p - b0, e - b0, DIM == 3 ? z % NS : 0, rec, cs, kp);
+            const int e = min(ke, b0 + B);
+            acc.accumulate(p - b0, e - b0, DIM == 3 ? z % NS : 0, rows, sh, cs);
             p = e;
         }
     }
@@ -499,14 +562,19 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
 // Interp (the product's inner dimension = (y, z) cells, 4 per instruction,
 // one for each quarter of the wave).  3D: quarter (a, b) holds the y cells
 // a HY .. and z cells b HZ ..; 2D: quarter q holds y = 4 i + q.  A wave takes
-// up to NB batches of 16 points of one window: it evaluates their y and z
-// weights in the operand layout of the product (each lane only those of its
-// own cells), reads the window's cells straight from the fine grid (a window is
+// up to NB batches of 16 points of one window: it takes their weights from LDS
+// in the operand layout of the product (each lane only those of its own
+// cells), reads the window's cells straight from the fine grid (a window is
 // read once per run; neighbouring windows share lines in L1 and L2) and
 // finishes with the x weights and a sum over 16 lanes.
-template <int DIM, int NS>
+template <typename T, int DIM, int NS>
 struct InterpWin {
     static constexpr int NB = DIM == 3 ? 2 : 4;
+    // points staged at a time, and held: two blocks, so that a run of 16 NB points
+    // may start anywhere, where 2 workgroups per CU (FP64) then still fit
+    static constexpr int block = 16 * NB;
+    static constexpr int ring =
+        DIM == 3 && WinRow<T, DIM, NS>::pitch * sizeof(T) * 4 * 64 <= 76 * 1024 ? 64 : block;
     static constexpr int HY = DIM == 2 ? 4 : win_interp_half(NS);
     static constexpr int HZ = DIM == 2 ? 1 : HY;
     static constexpr int SX = 17 - NS, SY = DIM == 2 ? 17 - NS : 2 * HY - NS + 1,
@@ -518,35 +586,39 @@ __device__ __forceinline__ void win_interp_run(int s, int npt, int gx, const int
                                                const long long *zo, int M, int ntr,
                                                cpx<T> *__restrict__ c,
                                                const cpx<T> *__restrict__ fw, long long nftot,
-                                               const KerParams<T> &kp, double back,
-                                               const WinRec<T> *rec, const int *ids)
+                                               double back, const T *rows, const unsigned *sh,
+                                               const int *ids)
 {
-    using W = InterpWin<DIM, NS>;
+    using W = InterpWin<T, DIM, NS>;
+    using Row = WinRow<T, DIM, NS>;
     using Acc = typename Mfma<T>::Acc;
     const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
-    const T hw = T(0.5) * NS;
     T ky[NB][W::HY], kz[NB][W::HZ], kx[NB][4];
     int dst[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const WinRec<T> r = rec[s + min(16 * b + i16, npt - 1)];
-        const T fy = (T)(DIM == 2 ? q : (q & 1) * W::HY) - hw - (T)(r.sh >> 8 & 255);
+        const int p = (s + min(16 * b + i16, npt - 1)) & (W::ring - 1);
+        const T *row = rows + __umul24(p, Row::pitch);
+        const unsigned u = sh[p];
+        const int y = (DIM == 2 ? q : (q & 1) * W::HY) - (int)(u >> 8 & 255);
 #pragma unroll
         for (int k = 0; k < W::HY; ++k)
-            ky[b][k] = win_phi(r.x[1] + (fy + (T)(DIM == 2 ? 4 * k : k)), kp);
+            ky[b][k] = row[Row::Y + Row::tap(y + (DIM == 2 ? 4 * k : k))];
         if (DIM == 3) {
-            const T fz = (T)((q >> 1) * W::HZ) - hw - (T)(r.sh >> 16 & 31);
+            // the z taps have no zero behind them: the one of y stands in
+            const int z = (q >> 1) * W::HZ - (int)(u >> 16);
 #pragma unroll
-            for (int k = 0; k < W::HZ; ++k) kz[b][k] = win_phi(r.x[2] + (fz + (T)k), kp);
+            for (int k = 0; k < W::HZ; ++k)
+                kz[b][k] = row[(unsigned)(z + k) < (unsigned)NS ? Row::Z + z + k : Row::Y + NS];
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const WinRec<T> &rk = rec[s + min(16 * b + mfma_row<T>(q, k), npt - 1)];
-            kx[b][k] = win_phi(rk.x[0] + ((T)i16 - hw - (T)(rk.sh & 255)), kp);
+            const int pk = (s + min(16 * b + mfma_row<T>(q, k), npt - 1)) & (W::ring - 1);
+            kx[b][k] = rows[__umul24(pk, Row::pitch) + Row::tap(i16 - (int)(sh[pk] & 255))];
         }
         // the lanes i16 < 4 of quarter q store the point of result row i16
         const int pd = 16 * b + mfma_row<T>(q, i16 & 3);
-        dst[b] = i16 < 4 && pd < npt ? ids[s + pd] : -1;
+        dst[b] = i16 < 4 && pd < npt ? ids[(s + pd) & (W::ring - 1)] : -1;
     }
     for (int t = 0; t < ntr; ++t) {
         const cpx<T> *f = fw + (long long)t * nftot + gx;
@@ -602,14 +674,17 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
 k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict__ fw, BinGeom g,
              WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
 {
-    using W = InterpWin<DIM, NS>;
+    using W = InterpWin<T, DIM, NS>;
+    using Row = WinRow<T, DIM, NS>;
     constexpr int F = (NS + 1) / 2 + 1;
-    __shared__ WinRec<T> srec[256];
-    __shared__ int sids[256];
+    __shared__ T srow[4 * W::ring * Row::pitch];
+    __shared__ unsigned ssh[4 * W::ring];
+    __shared__ int sids[4 * W::ring];
     const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    WinRec<T> *rec = srec + wave * 64;
-    int *ids = sids + wave * 64;
+    T *rows = srow + wave * W::ring * Row::pitch;
+    unsigned *sh = ssh + wave * W::ring;
+    int *ids = sids + wave * W::ring;
     const T *x1 = static_cast<const T *>(wp.x);
     const JobRange jr = xcd_jobs(gridDim.x);
     const int rng = (int)jr.begin * 4 + wave;
@@ -620,19 +695,38 @@ k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict_
     const double back = exp((double)DIM * (double)kp.beta);
     WinKeys keys;
     keys.load(wp, wg.nkeys, win_key_of(wp.start, wg.nkeys, p));
-    T xa[DIM];
+    Row::clear(rows, W::ring, lane);
+    // 3D: blocks of 32 points, lane l has point l % 32 and, half h of the wave,
+    // axis h and a half of the z weights.  2D: blocks of 64, both axes.  The next
+    // block is in flight while one is worked on.
+    const int h = DIM == 3 ? lane >> 5 : 0, pl = lane & (W::block - 1);
+    T xa[2];
     unsigned sa;
     int ia;
     auto load = [&](int i) {
         const int k = min(i, pe - 1);
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) xa[d] = x1[d * wp.stride + k];
+        xa[0] = x1[h * wp.stride + k];
+        xa[1] = x1[(DIM - 1) * wp.stride + k];
         sa = wp.sh[k];
         ia = wp.idx[k];
     };
-    load(p + lane);
-    int b0 = p;
-    bool staged = false;
+    int b0 = p, se = p;  // the range's first point, the staged points' end
+    auto stage = [&]() {
+        __builtin_amdgcn_wave_barrier();
+        const int at = (se - b0 + pl) & (W::ring - 1);
+        T *row = rows + at * Row::pitch;
+        Row::axis(row + h * Row::Y, xa[0], kp);
+        if (DIM == 3)
+            Row::half(row + Row::Z, h, xa[1], kp);
+        else
+            Row::axis(row + Row::Y, xa[1], kp);
+        sh[at] = sa;
+        ids[at] = ia;
+        se += W::block;
+        load(se + pl);
+        __builtin_amdgcn_wave_barrier();
+    };
+    load(p + pl);
     while (p < pe) {
         const int key = keys.key_of(wp, wg.nkeys, p);
         const int ke = min(pe, keys.key_end(key));
@@ -654,23 +748,14 @@ k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict_
                                   g.nf[1] * g.nf[0]
                             : 0;
         while (p < ke) {
-            if (!staged || p >= b0 + 64) {
-                if (staged) b0 += 64;
-                staged = true;
-                __builtin_amdgcn_wave_barrier();
-                WinRec<T> r;
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) r.x[d] = xa[d];
-                r.sh = sa;
-                rec[lane] = r;
-                ids[lane] = ia;
-                load(b0 + 64 + lane);
-                __builtin_amdgcn_wave_barrier();
-            }
-            const int npt = min(min(ke, b0 + 64) - p, 16 * W::NB);
+            int npt = min(ke - p, 16 * W::NB);
+            if (W::ring > W::block ? p + npt > se : p >= se) stage();
+            // (the first run of a range needs at most one block, a later one finds
+            // its first point's staged)
+            if (W::ring == W::block) npt = min(npt, se - p);
 #define CFA_RUN(NB)                                                                              \
-    win_interp_run<T, DIM, NS, NB>(p - b0, npt, gx, yo, zo, M, ntr, c, fw, nftot, kp, back, rec, \
-                                   ids)
+    win_interp_run<T, DIM, NS, NB>(p - b0, npt, gx, yo, zo, M, ntr, c, fw, nftot, back, rows,    \
+                                   sh, ids)
             if (npt <= 16)
                 CFA_RUN(1);
             else if (W::NB == 2 || npt <= 32)
