@@ -29,6 +29,7 @@ struct WinGeom {
     int nw[3] = {1, 1, 1};
     int nkeys = 0;
     int ns = 2;
+    bool ystrips = false;  // 2D keys run along y (see win_key)
     int ranges = 0;
 };
 // The points in window order, as the kernels read them.
@@ -37,9 +38,10 @@ struct WinPts {
     const unsigned *sh;   // first tap inside its window, a byte per axis
     const int *idx;       // the caller's index
     const int *start;     // first point of each window (nkeys + 1)
-    const int *range;     // first point of each range (ranges + 1)
+    const int2 *range;    // first point of each range (ranges + 1) and its window
     long long stride;
 };
+constexpr int kWinPack = 64;      // bytes of a point's packed strengths
 constexpr int kWinKeyWeight = 8;  // a window's own time in a range, in points
 // Half of a 3D interp window's y and z extent: windows of 8 cells up to ns 8,
 // of ns + 1 or ns + 2 beyond.
@@ -72,10 +74,11 @@ struct SortBufs {
     int *wstart = nullptr;     // [nkeys + 1]
     int *wused = nullptr;      // [nkeys + 1] windows with points before each
     void *wpart = nullptr;     // scan partials (int2) and totals
-    int *wrange = nullptr;     // [ranges + 1]
+    int2 *wrange = nullptr;    // [ranges + 1]
     void *wx = nullptr;        // T [dim][pos_stride]
     unsigned *wsh = nullptr;   // [M]
     int *widx = nullptr;       // [M]
+    void *wc = nullptr;        // kWinPack bytes a point: packed strengths of a 2D batch
     // method 4: point copies counted per block
     int *kcount = nullptr;       // [nkeys]
     int *kstart = nullptr;       // [nkeys]

@@ -725,7 +725,8 @@ struct Plan {
         dfree(sb.wrange);
         if (sb.wpart) hipFree(sb.wpart);
         if (sb.wx) hipFree(sb.wx);
-        sb.wpart = sb.wx = nullptr;
+        if (sb.wc) hipFree(sb.wc);
+        sb.wpart = sb.wx = sb.wc = nullptr;
         dfree(sb.wsh);
         dfree(sb.widx);
         cap_wkeys = cap_wM = cap_wranges = -1;
@@ -1086,6 +1087,12 @@ int Plan<T>::alloc_win()
         (void)hipGetLastError();
         free_win();
         return kErrHip;
+    }
+    // without it the spread gathers the strengths from the caller's array
+    if (dim == 2 && type == 1 && std::min(maxbatch, ntransf) >= 4 &&
+        hipMalloc(&sb.wc, (size_t)kWinPack * (size_t)sb.pos_stride) != hipSuccess) {
+        (void)hipGetLastError();
+        sb.wc = nullptr;
     }
     cap_wkeys = keys;
     cap_wranges = sb.win.ranges;

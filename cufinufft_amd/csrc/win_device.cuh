@@ -194,12 +194,14 @@ CFA_HD int win_wrap(int c, int n)
     return c - (c >= n ? n : 0);
 }
 
-// Key of a window: along z (3D) fastest, then x, then y, so a strip of windows
-// along z is a run of the order.
+// Key of a window.  3D: along z fastest, so a strip of windows along z is a run of
+// the order; 2D spread: along y for the same reason; 2D interp: along x, as the bins
+// (the window order of 3e6 FP64 points then takes 20 us less).
 template <int DIM>
 CFA_HD int win_key(const WinGeom &w, const int *k)
 {
-    return DIM == 3 ? (k[1] * w.nw[0] + k[0]) * w.nw[2] + k[2] : k[1] * w.nw[0] + k[0];
+    if (DIM == 3) return (k[1] * w.nw[0] + k[0]) * w.nw[2] + k[2];
+    return w.ystrips ? k[0] * w.nw[1] + k[1] : k[1] * w.nw[0] + k[0];
 }
 
 // Windows of a grid nf for transforms of the given type and width: S, nw, nkeys,
@@ -208,6 +210,7 @@ CFA_HD int win_key(const WinGeom &w, const int *k)
 inline bool win_windows(int type, int dim, int ns, const int *nf, WinGeom &w)
 {
     w.ns = ns;
+    w.ystrips = type == 1;
     w.S[0] = w.S[1] = 17 - ns;
     w.S[2] = 1;
     if (dim == 3 && type == 2) w.S[1] = w.S[2] = 2 * win_interp_half(ns) - ns + 1;
@@ -318,8 +321,13 @@ struct WinRow {
 // when the first plane moves on, the planes left behind go to the fine grid
 // with global atomics.  So a strip writes every cell of its 16 x 16 column
 // once: 256 / (17 - ns)^2 cells per grid cell (2.1 at ns 6), and no LDS tile, no
-// common scale and no barrier is needed.  In 2D a window is one such plane,
-// and NT transforms share the weights.
+// common scale and no barrier is needed.  In 2D a window is one such plane, the
+// strips run along y, row y is held in row slot y mod 16, and a window that follows
+// its neighbour takes over the ns - 1 rows they share (17 - ns rows are written
+// instead of 16); NT transforms share the weights.  Points come in window order, so strengths
+// are gathered, 8 or 16 bytes of each 64-byte piece: batches are first packed point
+// after point (k_win_pack; 32 coils of
+// 2e6 points on 1024^2, ns 7, in batches of 8: 1.56 -> 1.27 ms with the shared rows).
 //
 // Bounds per 4 points and SIMD: 64 ns (FP32) or 128 ns clocks of the matrix cores
 // in 3D, about 110 for the operands and 120 for the weights (which took 240 when
@@ -353,26 +361,29 @@ struct WinSpread {
         constexpr int S = 17 - NS, F = (NS + 1) / 2 + 1;
         const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            row[r] = 2u * (unsigned)(win_wrap(ky * S - F + q + 4 * r, g.nf[1]) * g.nf[0]);
+        for (int r = 0; r < 4; ++r) {
+            const int j = DIM == 2 ? (q + 4 * r - ky * S) & 15 : q + 4 * r;
+            row[r] = 2u * (unsigned)(win_wrap(ky * S - F + j, g.nf[1]) * g.nf[0]);
+        }
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             constexpr int cells = 32 / sizeof(T);  // cells of 64 bytes
-            const int at = kx * S - F + (ky * S - F + q) * g.nf[0];
+            const int at = kx * S - F + (DIM == 2 ? q - F : ky * S - F + q) * g.nf[0];
             src[b] = (unsigned)(16 * b + i16 - 2 * (at & (cells - 1))) & 31;
             col[b] = 2u * (unsigned)win_wrap(kx * S - F + (int)(src[b] >> 1), g.nf[0]) + (src[b] & 1);
         }
     }
-    // Points s .. e - 1 of the staged block (of one window); zslot: slot of their
-    // first plane.
-    __device__ __forceinline__ void accumulate(int s, int e, int zslot, const T *rows,
+    // Points s .. e - 1 of the staged block (of one window); slot: that of their
+    // first plane (3D) or of the window's first row (2D).
+    __device__ __forceinline__ void accumulate(int s, int e, int slot, const T *rows,
                                                const unsigned *sh, const cpx<T> *cs)
     {
         using Row = WinRow<T, DIM, NS>;
         const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
         // lane i of a row takes the x and y weights of cell i and the z weight
         // of slot i (any weight for i >= ns)
-        const int zt = i16 - zslot, z = Row::Z + min(zt < 0 ? zt + NS : zt, NS - 1);
+        const int zt = i16 - slot, z = Row::Z + min(zt < 0 ? zt + NS : zt, NS - 1);
+        const int y = DIM == 2 ? zt & 15 : i16;
         // quarter q of the wave holds point b + q; groups of 4 start at multiples
         // of 4 of the block, so only a window's first and last are not full
         for (int b = s & ~3; b < e; b += 4) {
@@ -381,13 +392,13 @@ struct WinSpread {
             const T *row = rows + __umul24(p, Row::pitch);
             const unsigned u = sh[p];
             const T kx = row[ok ? Row::tap(i16 - (int)(u & 255)) : NS];
-            const T ky = row[Row::Y + Row::tap(i16 - (int)(u >> 8 & 255))];
+            const T ky = row[Row::Y + Row::tap(y - (int)(u >> 8 & 255))];
             T kz = T(0);
             if (DIM == 3) kz = row[z];
             T br[NT], bi[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const cpx<T> v = cs[kBlock * t + p];
+                const cpx<T> v = cs[NT * p + t];
                 br[t] = v.x * kx;
                 bi[t] = v.y * kx;
             }
@@ -402,16 +413,18 @@ struct WinSpread {
             });
         }
     }
-    // Adds plane slot m of every transform to the grid and clears it; plane: the
-    // plane's first cell in transform 0.  The lanes first trade places through
+    // Adds plane slot m (2D: the first `rows` rows, from slot `slot` on) of every
+    // transform to the grid and clears it; plane: the plane's first cell in transform
+    // 0.  The lanes first trade places through
     // LDS (sc, 256 complex values of the wave), so that 16 lanes add the 16
     // components of 8 neighbouring cells: 1.9e11 adds per second against 1.2e11
     // for a lane per cell that adds its two components in turn (16 x 16 windows
     // every 10 cells of a 1024^2 FP32 grid).
     template <int m>
-    __device__ __forceinline__ void flush(T *plane, long long tstride, int nt, cpx<T> *sc)
+    __device__ __forceinline__ void flush(T *plane, long long tstride, int nt, cpx<T> *sc, int slot,
+                                          int rows)
     {
-        const int lane = threadIdx.x & 63;
+        const int lane = threadIdx.x & 63, q = lane >> 4;
         // row q + 4 r: register r of quarter q in FP64, register q of quarter r in FP32
         const T *from = reinterpret_cast<const T *>(sc) + (lane >> 4) * (sizeof(T) == 4 ? 128 : 32);
 #pragma unroll
@@ -428,30 +441,54 @@ struct WinSpread {
                 }
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
+                for (int r = 0; r < 4; ++r) {
+                    if (DIM == 2 && ((q + 4 * r - slot) & 15) >= rows) continue;
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
                         const T v = from[(sizeof(T) == 4 ? 32 : 128) * r + src[b]];
                         if (v != T(0)) gadd(p + (row[r] + col[b]), v);
                     }
+                }
             }
-            ar[t][m] = ai[t][m] = Acc{0, 0, 0, 0};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (DIM == 3 || ((mfma_row<T>(q, r) - slot) & 15) < rows)
+                    ar[t][m][r] = ai[t][m][r] = T(0);
         }
     }
 };
 
+// Strengths of NT transforms, point after point: out[NT i + t] = c[t M + i].
+template <typename T, int NT>
+__global__ void __launch_bounds__(256)
+k_win_pack(int M, int nt, const cpx<T> *__restrict__ c, cpx<T> *__restrict__ out)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= M) return;
+    cpx<T> v[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        v[t].x = v[t].y = T(0);
+        if (t < nt) v[t] = c[(long long)t * M + i];
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) out[(long long)NT * i + t] = v[t];
+}
+
+// Point id's strength of transform t is c[t ct + id ci].
 template <typename T, int DIM, int NS, int NT>
 __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
-k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict__ fw, BinGeom g,
-             WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
+k_win_spread(WinPts wp, const cpx<T> *__restrict__ c, long long ct, int ci, cpx<T> *__restrict__ fw,
+             BinGeom g, WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
 {
-    constexpr int F = (NS + 1) / 2 + 1;
+    constexpr int F = (NS + 1) / 2 + 1, S = 17 - NS;
     using Acc = WinSpread<T, DIM, NS, NT>;
     using Row = WinRow<T, DIM, NS>;
     constexpr int B = Acc::kBlock;
     __shared__ T srow[4 * B * Row::pitch];
     __shared__ unsigned ssh[4 * B];
-    __shared__ cpx<T> scs[4 * B * NT], ssc[1024];
+    __shared__ alignas(16) cpx<T> scs[4 * B * NT];
+    __shared__ cpx<T> ssc[1024];
     const int lane = threadIdx.x & 63, h = lane >> 5, pl = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     T *rows = srow + wave * B * Row::pitch;
@@ -461,20 +498,21 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
     const JobRange jr = xcd_jobs(gridDim.x);  // one range per wave, contiguous per XCD
     const int rng = (int)jr.begin * 4 + wave;
     if (rng >= wg.ranges) return;
-    int p = wp.range[rng];
-    const int pe = wp.range[rng + 1];
+    const int2 r0 = wp.range[rng];
+    int p = r0.x;
+    const int pe = wp.range[rng + 1].x;
     if (p >= pe) return;
     const int t0 = blockIdx.y * NT, nt = min(NT, ntr - t0);
-    c += (long long)t0 * M;
+    c += t0 * ct;
     T *ft = reinterpret_cast<T *>(fw + (long long)t0 * nftot);
     const double back = exp((double)DIM * (double)kp.beta);
     Acc acc;
     acc.clear();
     Row::clear(rows, B, lane);
     WinKeys keys;
-    keys.load(wp, wg.nkeys, win_key_of(wp.start, wg.nkeys, p));
+    keys.load(wp, wg.nkeys, r0.y);
     // blocks of 32 points: lane l has point l % 32 and, half h of the wave, axis h
-    // (and a half of the z weights), and the transforms t = h mod 2.  The next
+    // (and a half of the z weights), and a half of the transforms.  The next
     // block's strengths and the records of the one after are in flight while one
     // is worked on
     constexpr int NC = (NT + 1) / 2;
@@ -493,9 +531,9 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
     auto gather = [&](int id) {
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
-            const int t = 2 * j + h;
+            const int t = NC * h + j;
             ca[j].x = ca[j].y = T(0);
-            if (t < nt) ca[j] = c[(long long)t * M + id];
+            if (t < nt) ca[j] = c[t * ct + (long long)id * ci];
         }
     };
     load(p + pl, xa, za, sa, ib);
@@ -503,8 +541,8 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
     load(p + B + pl, xb, zb, sb, ib);
     int b0 = p;
     bool staged = false;
-    int strip = -1, z = 0;  // window held (3D: its first plane's place too)
-    const int nz = DIM == 3 ? wg.nw[2] : 1;
+    int strip = -1, z = 0;  // strip of the points held and the window's place in it
+    const int nz = wg.nw[DIM - 1];
     const long long pstride = 2ll * g.nf[0] * g.nf[1];
     for (;;) {
         const bool last = p >= pe;
@@ -512,21 +550,28 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
         if (!last) {
             key = keys.key_of(wp, wg.nkeys, p);
             ke = min(pe, keys.key_end(key));
-            st = DIM == 3 ? key / nz : key;
-            zk = DIM == 3 ? key - st * nz : 0;
+            st = key / nz;
+            zk = key - st * nz;
         }
-        // the planes no later point of the strip reaches go to the grid
-        const int nf = strip < 0 ? 0 : (st != strip ? acc.RB : min(zk - z, acc.RB));
-        for (int k = z; k < z + nf; ++k) {
-            T *plane = ft + (DIM == 3 ? win_wrap(k - F, g.nf[2]) * pstride : 0);
-            const int m = DIM == 3 ? k % NS : 0;
-            static_for<Acc::RB>([&](auto mc) {
-                if (m == decltype(mc)::value)
-                    acc.template flush<decltype(mc)::value>(plane, 2 * nftot, nt, sc);
-            });
+        // the planes (2D: rows) no later point of the strip reaches go to the grid
+        if (DIM == 3) {
+            const int nf = strip < 0 ? 0 : (st != strip ? NS : min(zk - z, NS));
+            for (int k = z; k < z + nf; ++k) {
+                T *plane = ft + win_wrap(k - F, g.nf[2]) * pstride;
+                const int m = k % NS;
+                static_for<Acc::RB>([&](auto mc) {
+                    if (m == decltype(mc)::value)
+                        acc.template flush<decltype(mc)::value>(plane, 2 * nftot, nt, sc, 0, 16);
+                });
+            }
+            if (st != strip && !last) acc.place(st % wg.nw[0], st / wg.nw[0], g);
+        } else {
+            if (strip >= 0)
+                acc.template flush<0>(ft, 2 * nftot, nt, sc, z * S & 15,
+                                      st != strip ? 16 : min((zk - z) * S, 16));
+            if (!last) acc.place(st, zk, g);
         }
         if (last) break;
-        if (st != strip) acc.place(st % wg.nw[0], st / wg.nw[0], g);
         strip = st;
         z = zk;
         while (p < ke) {
@@ -542,7 +587,7 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
                 for (int j = 0; j < NC; ++j) {
                     ca[j].x = (T)((double)ca[j].x * back);
                     ca[j].y = (T)((double)ca[j].y * back);
-                    if (2 * j + h < NT) cs[B * (2 * j + h) + pl] = ca[j];
+                    if (NC * h + j < NT) cs[NT * pl + NC * h + j] = ca[j];
                 }
                 gather(ib);
                 xa = xb;
@@ -552,7 +597,7 @@ k_win_spread(int M, WinPts wp, const cpx<T> *__restrict__ c, cpx<T> *__restrict_
                 __builtin_amdgcn_wave_barrier();
             }
             const int e = min(ke, b0 + B);
-            acc.accumulate(p - b0, e - b0, DIM == 3 ? z % NS : 0, rows, sh, cs);
+            acc.accumulate(p - b0, e - b0, DIM == 3 ? z % NS : z * S & 15, rows, sh, cs);
             p = e;
         }
     }
@@ -689,12 +734,13 @@ k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict_
     const JobRange jr = xcd_jobs(gridDim.x);
     const int rng = (int)jr.begin * 4 + wave;
     if (rng >= wg.ranges) return;
-    int p = wp.range[rng];
-    const int pe = wp.range[rng + 1];
+    const int2 r0 = wp.range[rng];
+    int p = r0.x;
+    const int pe = wp.range[rng + 1].x;
     if (p >= pe) return;
     const double back = exp((double)DIM * (double)kp.beta);
     WinKeys keys;
-    keys.load(wp, wg.nkeys, win_key_of(wp.start, wg.nkeys, p));
+    keys.load(wp, wg.nkeys, r0.y);
     Row::clear(rows, W::ring, lane);
     // 3D: blocks of 32 points, lane l has point l % 32 and, half h of the wave,
     // axis h and a half of the z weights.  2D: blocks of 64, both axes.  The next

@@ -1,5 +1,7 @@
 // Runtime-ns dispatch of the window kernels for one (T, DIM); included by the
 // win_spread_<prec><dim>.hip and win_interp_<prec><dim>.hip translation units.
+#include <algorithm>
+
 #include "nufft_launch.h"
 #include "win_device.cuh"
 
@@ -26,13 +28,24 @@ int win_spread_ns(int M, const SortBufs &sb, const cpx<T> *c, cpx<T> *fw, const 
         return 1;
     } else {
         const int grid = win_grid(sb.win);
-        if (DIM == 2 && ntr > 1)
+        constexpr int P = DIM == 2 ? kWinPack / (int)sizeof(cpx<T>) : 1;
+        if (DIM == 2 && ntr >= 4 && sb.wc) {
+            cpx<T> *pk = static_cast<cpx<T> *>(sb.wc);
+            for (int t = 0; t < ntr; t += P) {
+                const int nt = std::min(P, ntr - t);
+                k_win_pack<T, P><<<(M + 255) / 256, 256, 0, L.stream>>>(M, nt,
+                                                                        c + (long long)t * M, pk);
+                k_win_spread<T, DIM, NS, P><<<grid, 256, 0, L.stream>>>(
+                    win_pts(sb), pk, 1, P, fw + t * nftot, g, sb.win, kp, nt, nftot);
+            }
+        } else if (DIM == 2 && ntr > 1) {
             k_win_spread<T, DIM, NS, DIM == 2 ? 4 : 1>
-                <<<dim3(grid, (ntr + 3) / 4), 256, 0, L.stream>>>(M, win_pts(sb), c, fw, g, sb.win,
-                                                                  kp, ntr, nftot);
-        else
+                <<<dim3(grid, (ntr + 3) / 4), 256, 0, L.stream>>>(win_pts(sb), c, M, 1, fw, g,
+                                                                  sb.win, kp, ntr, nftot);
+        } else {
             k_win_spread<T, DIM, NS, 1><<<dim3(grid, ntr), 256, 0, L.stream>>>(
-                M, win_pts(sb), c, fw, g, sb.win, kp, ntr, nftot);
+                win_pts(sb), c, M, 1, fw, g, sb.win, kp, ntr, nftot);
+        }
         return hipGetLastError() == hipSuccess ? 0 : kErrHip;
     }
 }

@@ -92,11 +92,14 @@ k_win_keys(int M, SortedPts sp, WinGeom wg, int *__restrict__ count,
 
 static __global__ void __launch_bounds__(256)
 k_win_ranges(int M, int nkeys, int ranges, int *__restrict__ start, const int *__restrict__ used,
-             int *__restrict__ range)
+             int2 *__restrict__ range)
 {
     const int r = blockIdx.x * 256 + threadIdx.x;
     if (r == 0) start[nkeys] = M;
-    if (r <= ranges) range[r] = win_range_start(start, used, nkeys, M, r, ranges);
+    if (r <= ranges) {
+        const int p = win_range_start(start, used, nkeys, M, r, ranges);
+        range[r] = make_int2(p, win_key_of(start, nkeys, p));
+    }
 }
 
 // Where the window kernels beat the per-point ones, the window order's own time
@@ -136,9 +139,13 @@ WinGeom win_choose(int type, int dim, int ns, int elem, const BinGeom &g, int M,
     // One wave per range.  Interp: up to 8 rounds of the waves resident on the
     // device (16 per CU FP32, 8 FP64), no fewer than 128 points each.  Spread: a
     // range flushes a whole window at its end, so ranges grow to 1536 points before
-    // there are more than half a round of them, and stop at 4 rounds.
+    // there are more than half a round of them, and stop at 4 rounds.  2D spread:
+    // one round (half a round: 0.326 -> 0.298 ms, FP32, ns 7, 1e7 points; two rounds
+    // cost 32 coils of 2e6 points 1.27 -> 1.49 ms in flushes).
     const int resident = ncu * (elem == 4 ? 16 : 8);
-    if (type == 2)
+    if (dim == 2 && type == 1)
+        w.ranges = std::max(1, std::min(resident, M / 128));
+    else if (type == 2)
         w.ranges = std::max(1, std::min(8 * resident, M / 128));
     else
         w.ranges = std::max({1, std::min(resident / 2, M / 128),

@@ -133,3 +133,24 @@ def test_window_changing_points(torch_dev):
         torch.cuda.synchronize()
         if M != 500:
             assert rel_l2(fk.cpu().numpy(), P.type1(pts, c)) < 5e-7
+
+
+@pytest.mark.parametrize("dtype,ns,ntr,M", [(F32, 7, 4, 1100000), (F32, 7, 7, 600000),
+                                            (F32, 8, 13, 300000), (F64, 9, 6, 210000),
+                                            (F64, 13, 4, 160000)])
+def test_window_packed_batch(torch_dev, dtype, ns, ntr, M):
+    """Packed strengths of 2D batches, whole and partly filled packs, on points that
+    leave gaps of one and more windows along y (rows taken over, or all flushed)."""
+    print(f"window batch {dtype} {ns} {ntr}", flush=True)
+    nm, tol, single = (40, 66), _tol(dtype, ns), dtype == F32
+    pts = _pts(2, M, dtype, [2 * n for n in nm], 5)
+    u = pts[1].astype(np.float64) / (2 * np.pi) + 0.5  # bands of y: 0.1, a gap of 0.06, ...
+    u = np.where((u > 0.1) & (u < 0.16), 0.05, np.where((u > 0.4) & (u < 0.65), 0.7, u))
+    pts[1] = ((u - 0.5) * (2 * np.pi)).astype(dtype)
+    P = O.Plan(1, list(nm), tol, single=single)
+    c = G.strengths(M, dtype, 5, ntr)
+    got, _ = G.run_type1(torch_dev, pts, c, nm, tol, dtype, ntr, maxbatchsize=ntr)
+    bar = max(tol / 5, 5e-7 if single else 1e-13)
+    for t in range(ntr):
+        ref = P.type1(pts, c.reshape(ntr, M)[t])
+        assert rel_l2(got.reshape(ntr, -1)[t], ref) < bar
