@@ -19,8 +19,8 @@
 // clock and CU for 32-bit, 64-bit integer and FP64 LDS adds), the per-point
 // interp one LDS or L1 read and two FMAs per tap.
 // Spread or interp alone, per-point -> window kernel: 3D FP32 type 1, ns 6, 1e8
-// points on 512^3: 20.7 -> 6.9 ms; 3D FP64 type 2, ns 10, 1e7: 17.7 -> 3.3 ms;
-// 2D FP64 type 2: 0.90 -> 0.35 ms (the rule of win_sort.hip has both sides at
+// points on 512^3: 20.7 -> 6.9 ms; 3D FP64 type 2, ns 10, 1e7: 17.7 -> 2.5 ms;
+// 2D FP64 type 2: 0.90 -> 0.30 ms (the rule of win_sort.hip has both sides at
 // the edges of its range).
 #pragma once
 #include <utility>
@@ -57,37 +57,21 @@ __device__ __forceinline__ int mfma_row(int q, int r)
 }
 
 // Lane movement inside rows of 16 lanes (DPP); CTRL as in the ISA's dpp_ctrl:
-// 0x150 + n broadcasts lane n of each row, 0x120 + n rotates right by n, 0x100 +
-// n / 0x110 + n shift by n lanes down / up, 0x55 n broadcasts lane n of each quad.
-// Lanes whose bank (4 lanes) is not in BANKS keep old.
-template <int CTRL, int BANKS>
-__device__ __forceinline__ float dpp(float old, float v)
+// broadcast of lane n of each row (0x150 + n), rotation by n (0x120 + n), lane i from
+// lane 7 - i of each 8, from lane i ^ 1 and i ^ 2.
+constexpr int kDppBcast = 0x150, kDppRor = 0x120, kDppHalfMirror = 0x141, kDppQuadXor1 = 0xb1,
+              kDppQuadXor2 = 0x4e;
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v)
 {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL,
-                                                      0xf, BANKS, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-template <int CTRL, int BANKS>
-__device__ __forceinline__ double dpp(double old, double v)
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf,
-                                               BANKS, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf,
-                                               BANKS, false);
-    return __hiloint2double(hi, lo);
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
 }
-// Broadcast of lane N of each row.
-template <int N>
-__device__ __forceinline__ float row_bcast(float v)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + N, 0xf, 0xf, true));
-}
-template <int N>
-__device__ __forceinline__ double row_bcast(double v)
-{
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + N, 0xf, 0xf, true),
-                            __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + N, 0xf, 0xf, true));
-}
-constexpr int kDppBcast = 0x150, kDppRor = 0x120, kDppShl = 0x100, kDppShr = 0x110;
 
 // f(0), ..., f(N - 1) with the index as a compile-time constant.
 template <class F, int... I>
@@ -99,17 +83,6 @@ template <int N, class F>
 __device__ __forceinline__ void static_for(F &&f)
 {
     static_for_seq(f, std::make_integer_sequence<int, N>{});
-}
-
-// Sum over each row of 16 lanes, in every lane.
-template <typename T>
-__device__ __forceinline__ T row_sum(T v)
-{
-    v += dpp<kDppRor + 8, 0xf>(v, v);
-    v += dpp<kDppRor + 4, 0xf>(v, v);
-    v += dpp<kDppRor + 2, 0xf>(v, v);
-    v += dpp<kDppRor + 1, 0xf>(v, v);
-    return v;
 }
 
 // Square root of a in [2^-60, 1], within an ulp: the hardware reciprocal square
@@ -404,7 +377,7 @@ struct WinSpread {
             }
             static_for<RB>([&](auto mc) {
                 constexpr int m = decltype(mc)::value;
-                const T a = DIM == 3 ? ky * row_bcast<m>(kz) : ky;
+                const T a = DIM == 3 ? ky * dpp_mov<kDppBcast + m>(kz) : ky;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     ar[t][m] = Mfma<T>::mac(a, br[t], ar[t][m]);
@@ -622,14 +595,57 @@ struct InterpWin {
         DIM == 3 && WinRow<T, DIM, NS>::pitch * sizeof(T) * 4 * 64 <= 76 * 1024 ? 64 : block;
     static constexpr int HY = DIM == 2 ? 4 : win_interp_half(NS);
     static constexpr int HZ = DIM == 2 ? 1 : HY;
+    // planes of cells in flight: all of a window where registers allow
+    static constexpr int PF = DIM == 2 ? 1 : sizeof(T) == 4 || HZ == 4 ? HZ : 3;
     static constexpr int SX = 17 - NS, SY = DIM == 2 ? 17 - NS : 2 * HY - NS + 1,
                          SZ = DIM == 2 ? 1 : 2 * HZ - NS + 1;
 };
 
-template <typename T, int DIM, int NS, int NB>
-__device__ __forceinline__ void win_interp_run(int s, int npt, int gx, const int *yo,
-                                               const long long *zo, int M, int ntr,
-                                               cpx<T> *__restrict__ c,
+template <typename T>
+__device__ __forceinline__ cpx<T> load_cell(const __attribute__((address_space(1))) cpx<T> *p)
+{
+    cpx<T> v;
+    v.x = p->x;
+    v.y = p->y;
+    return v;
+}
+
+// A window's cells as a lane reads them: first cell (y0, z0) of the window, the
+// lane's own column gx, and for a window that does not wrap (inner) the lane's byte
+// offset from the window's first row, so that an address is the offset plus a sum
+// that the wave shares.
+struct WinBox {
+    int gx, y0, z0;
+    unsigned off;
+    bool inner;
+};
+
+// Sum of each of v[0..7] over a row of 16 lanes: lane i gets that of v[i / 2].  Each
+// step halves the values a lane carries: it keeps one half, gives the other to the
+// lane across (15 adds and 14 selects instead of 32 adds).
+template <typename T>
+__device__ __forceinline__ T row_sum8(const T *v)
+{
+    const int i = threadIdx.x;
+    T a[4], b[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const T keep = i & 8 ? v[j + 4] : v[j], give = i & 8 ? v[j] : v[j + 4];
+        a[j] = keep + dpp_mov<kDppRor + 8>(give);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const T keep = i & 4 ? a[j + 2] : a[j], give = i & 4 ? a[j] : a[j + 2];
+        b[j] = keep + dpp_mov<kDppHalfMirror>(give);
+    }
+    const T keep = i & 2 ? b[1] : b[0], give = i & 2 ? b[0] : b[1];
+    const T r = keep + dpp_mov<kDppQuadXor2>(give);
+    return r + dpp_mov<kDppQuadXor1>(r);
+}
+
+template <typename T, int DIM, int NS, int NB, bool INNER>
+__device__ __forceinline__ void win_interp_run(int s, int npt, const WinBox &w, const BinGeom &g,
+                                               int M, int ntr, cpx<T> *__restrict__ c,
                                                const cpx<T> *__restrict__ fw, long long nftot,
                                                double back, const T *rows, const unsigned *sh,
                                                const int *ids)
@@ -637,85 +653,130 @@ __device__ __forceinline__ void win_interp_run(int s, int npt, int gx, const int
     using W = InterpWin<T, DIM, NS>;
     using Row = WinRow<T, DIM, NS>;
     using Acc = typename Mfma<T>::Acc;
-    const int lane = threadIdx.x & 63, q = lane >> 4, i16 = lane & 15;
-    T ky[NB][W::HY], kz[NB][W::HZ], kx[NB][4];
-    int dst[NB];
+    constexpr int HY = W::HY, HZ = W::HZ, PF = W::PF;
+    // the empty asm statements keep the compiler from forming addresses and lane
+    // numbers ahead of the loops, which it would then spill
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int q = lane >> 4, i16 = lane & 15;
+    int nx = g.nf[0];
+    asm volatile("" : "+s"(nx));
+    constexpr int E = sizeof(cpx<T>);
+    const long long plane = (long long)nx * g.nf[1];
+    // (address space 1: global memory, which the statements would hide)
+    using Bytes = const __attribute__((address_space(1))) char *;
+    using Cells = const __attribute__((address_space(1))) cpx<T> *;
+    Bytes ft = (Bytes)(fw), pl;  // transform, next plane
+    if (INNER) ft += (w.z0 * plane + (long long)w.y0 * nx) * E;
+    unsigned row[HY];
+#pragma unroll
+    for (int k = 0; k < HY; ++k) row[k] = w.off + k * (DIM == 2 ? 4 : 1) * (unsigned)nx * E;
+    cpx<T> v[PF][HY];
+    // plane kk (2D: the rows) of the transform at ft
+    auto load = [&](int kk) {
+        if (INNER) {
+            pl = kk ? pl + plane * E : ft;
+            asm volatile("" : "+s"(pl));
+#pragma unroll
+            for (int k = 0; k < HY; ++k)
+                v[kk % PF][k] = load_cell<T>((Cells)(pl + row[k]));
+        } else {
+            int y0 = w.y0;
+            asm volatile("" : "+s"(y0));
+            const int z = DIM == 3 ? win_wrap(w.z0 + (q >> 1) * HZ + kk, g.nf[2]) : 0;
+            const Cells f = (Cells)ft + z * plane + w.gx;
+#pragma unroll
+            for (int k = 0; k < HY; ++k)
+                v[kk % PF][k] = load_cell<T>(f + (long long)nx * win_wrap(
+                    y0 + (DIM == 2 ? 4 * k + q : (q & 1) * HY + k), g.nf[1]));
+        }
+    };
+#pragma unroll
+    for (int kk = 0; kk < PF; ++kk) load(kk);
+    T ky[NB][HY], kz[NB][HZ];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         const int p = (s + min(16 * b + i16, npt - 1)) & (W::ring - 1);
         const T *row = rows + __umul24(p, Row::pitch);
         const unsigned u = sh[p];
-        const int y = (DIM == 2 ? q : (q & 1) * W::HY) - (int)(u >> 8 & 255);
+        const int y = (DIM == 2 ? q : (q & 1) * HY) - (int)(u >> 8 & 255);
 #pragma unroll
-        for (int k = 0; k < W::HY; ++k)
-            ky[b][k] = row[Row::Y + Row::tap(y + (DIM == 2 ? 4 * k : k))];
+        for (int k = 0; k < HY; ++k) ky[b][k] = row[Row::Y + Row::tap(y + (DIM == 2 ? 4 * k : k))];
         if (DIM == 3) {
             // the z taps have no zero behind them: the one of y stands in
-            const int z = (q >> 1) * W::HZ - (int)(u >> 16);
+            const int z = (q >> 1) * HZ - (int)(u >> 16);
 #pragma unroll
-            for (int k = 0; k < W::HZ; ++k)
+            for (int k = 0; k < HZ; ++k)
                 kz[b][k] = row[(unsigned)(z + k) < (unsigned)NS ? Row::Z + z + k : Row::Y + NS];
         }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int pk = (s + min(16 * b + mfma_row<T>(q, k), npt - 1)) & (W::ring - 1);
-            kx[b][k] = rows[__umul24(pk, Row::pitch) + Row::tap(i16 - (int)(sh[pk] & 255))];
-        }
-        // the lanes i16 < 4 of quarter q store the point of result row i16
-        const int pd = 16 * b + mfma_row<T>(q, i16 & 3);
-        dst[b] = i16 < 4 && pd < npt ? ids[(s + pd) & (W::ring - 1)] : -1;
     }
     for (int t = 0; t < ntr; ++t) {
-        const cpx<T> *f = fw + (long long)t * nftot + gx;
         // keep the ky kz products inside the loop over transforms (hoisted
         // out of it they would take HY HZ registers per batch)
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int k = 0; k < W::HY; ++k) asm volatile("" : "+v"(ky[b][k]));
+            for (int k = 0; k < HY; ++k) asm volatile("" : "+v"(ky[b][k]));
         Acc ar[NB], ai[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) ar[b] = ai[b] = Acc{0, 0, 0, 0};
-        // one plane of cells in flight while the one before is multiplied
-        cpx<T> v[2][W::HY];
+        // PF planes of cells in flight ahead of the one that is multiplied
 #pragma unroll
-        for (int k = 0; k < W::HY; ++k) v[0][k] = f[(DIM == 3 ? zo[0] : 0) + yo[k]];
+        for (int kk = 0; kk < HZ; ++kk) {
 #pragma unroll
-        for (int kk = 0; kk < W::HZ; ++kk) {
-            if (kk + 1 < W::HZ)
-#pragma unroll
-                for (int k = 0; k < W::HY; ++k) v[(kk + 1) & 1][k] = f[zo[kk + 1] + yo[k]];
-#pragma unroll
-            for (int k = 0; k < W::HY; ++k)
+            for (int k = 0; k < HY; ++k)
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
                     const T a = DIM == 3 ? ky[b][k] * kz[b][kk] : ky[b][k];
-                    ar[b] = Mfma<T>::mac(a, v[kk & 1][k].x, ar[b]);
-                    ai[b] = Mfma<T>::mac(a, v[kk & 1][k].y, ai[b]);
+                    ar[b] = Mfma<T>::mac(a, v[kk % PF][k].x, ar[b]);
+                    ai[b] = Mfma<T>::mac(a, v[kk % PF][k].y, ai[b]);
                 }
+            if (kk + PF < HZ) load(kk + PF);
             __builtin_amdgcn_sched_barrier(0);
         }
+        ft += nftot * E;
+        if (t + 1 < ntr)
+#pragma unroll
+            for (int kk = 0; kk < PF; ++kk) load(kk);
+        // the x weights, and the sums over the cells of a row: lane i of quarter q
+        // gets component (i / 2) % 2 of result row i / 4
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            cpx<T> o;
-            o.x = o.y = T(0);
+            int p[4];
+            unsigned u[4];
+            T r[8];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const T sr = row_sum(ar[b][k] * kx[b][k]), si = row_sum(ai[b][k] * kx[b][k]);
-                o.x = i16 == k ? sr : o.x;
-                o.y = i16 == k ? si : o.y;
+                p[k] = (s + min(16 * b + mfma_row<T>(q, k), npt - 1)) & (W::ring - 1);
+                u[k] = sh[p[k]];
             }
-            o.x = (T)((double)o.x * back);
-            o.y = (T)((double)o.y * back);
-            if (dst[b] >= 0) c[(long long)t * M + dst[b]] = o;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const T kx = rows[__umul24(p[k], Row::pitch) + Row::tap(i16 - (int)(u[k] & 255))];
+                r[2 * k] = ar[b][k] * kx;
+                r[2 * k + 1] = ai[b][k] * kx;
+            }
+            const T o = (T)((double)row_sum8(r) * back);
+            const int pd = 16 * b + mfma_row<T>(q, i16 >> 2);
+            if (!(i16 & 1) && pd < npt)
+                reinterpret_cast<T *>(c + (long long)t * M + ids[(s + pd) & (W::ring - 1)])
+                    [i16 >> 1 & 1] = o;
         }
     }
 }
 
 // Workgroups of 4 independent waves, one range of the order each; each XCD takes
 // a contiguous part of it.
+//
+// Bounds per 16 points: 64 HY HZ (FP32) or 128 HY HZ clocks of the matrix cores for
+// each transform, 1500 and more of the VALU, and below a few points per window the
+// latency of its cells: all their loads are in flight at once, from addresses that
+// the wave shares but for one offset per row.  That, the sums by row_sum8 and 3
+// FP32 workgroups per CU instead of 4 that spill took two FP32 volumes of 160^3, 4e6
+// points, ns 6, from 1.85 to 1.20 ms, 1e7 clustered FP64 points, ns 10, from 3.27
+// to 2.46 ms and 3e6 2D FP64 points, ns 13, from 0.35 to 0.30 ms.
 template <typename T, int DIM, int NS>
-__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 3 : 2)
 k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict__ fw, BinGeom g,
              WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
 {
@@ -779,29 +840,32 @@ k_win_interp(int M, WinPts wp, cpx<T> *__restrict__ c, const cpx<T> *__restrict_
         const int st = DIM == 3 ? key / wg.nw[2] : key;
         const int kz = DIM == 3 ? key - st * wg.nw[2] : 0;
         const int ky = st / wg.nw[0], kx = st - ky * wg.nw[0];
-        // the window's cells of this lane on the periodic grid
-        const int gx = win_wrap(kx * W::SX - F + i16, g.nf[0]);
-        int yo[W::HY];
-        long long zo[W::HZ];
-#pragma unroll
-        for (int j = 0; j < W::HY; ++j)
-            yo[j] = win_wrap(ky * W::SY - F + (DIM == 2 ? 4 * j + q : (q & 1) * W::HY + j),
-                             g.nf[1]) *
-                    g.nf[0];
-#pragma unroll
-        for (int j = 0; j < W::HZ; ++j)
-            zo[j] = DIM > 2 ? (long long)win_wrap(kz * W::SZ - F + (q >> 1) * W::HZ + j, g.nf[2]) *
-                                  g.nf[1] * g.nf[0]
-                            : 0;
+        WinBox w;
+        w.y0 = ky * W::SY - F;
+        w.z0 = DIM == 3 ? kz * W::SZ - F : 0;
+        w.gx = win_wrap(kx * W::SX - F + i16, g.nf[0]);
+        const long long plane = (long long)g.nf[0] * g.nf[1];
+        w.inner = w.y0 >= 0 && w.y0 + (DIM == 2 ? 16 : 2 * W::HY) <= g.nf[1] &&
+                  (DIM == 2 ? g.nf[0] < 1 << 24  // offsets fit 32 bits
+                            : w.z0 >= 0 && w.z0 + 2 * W::HZ <= g.nf[2] && plane < 1 << 25);
+        w.off = (unsigned)((w.gx + (DIM == 2 ? q : (q & 1) * W::HY) * (long long)g.nf[0] +
+                            (DIM == 3 ? (q >> 1) * W::HZ * plane : 0)) *
+                           (long long)sizeof(cpx<T>));
         while (p < ke) {
             int npt = min(ke - p, 16 * W::NB);
             if (W::ring > W::block ? p + npt > se : p >= se) stage();
             // (the first run of a range needs at most one block, a later one finds
             // its first point's staged)
             if (W::ring == W::block) npt = min(npt, se - p);
-#define CFA_RUN(NB)                                                                              \
-    win_interp_run<T, DIM, NS, NB>(p - b0, npt, gx, yo, zo, M, ntr, c, fw, nftot, back, rows,    \
-                                   sh, ids)
+#define CFA_RUN(NB)                                                                                \
+    do {                                                                                         \
+        if (w.inner)                                                                             \
+            win_interp_run<T, DIM, NS, NB, true>(p - b0, npt, w, g, M, ntr, c, fw, nftot, back,  \
+                                                 rows, sh, ids);                                 \
+        else                                                                                     \
+            win_interp_run<T, DIM, NS, NB, false>(p - b0, npt, w, g, M, ntr, c, fw, nftot, back, \
+                                                  rows, sh, ids);                                \
+    } while (0)
             if (npt <= 16)
                 CFA_RUN(1);
             else if (W::NB == 2 || npt <= 32)
