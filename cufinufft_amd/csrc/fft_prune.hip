@@ -38,17 +38,16 @@ template <typename T> constexpr int prune_w() { return sizeof(T) == 4 ? 64 : 32;
 // the axis) and c' - kneg otherwise; s = 1 / (kr[|r-hr|] kp[|p-hp|] kc[|c'-kneg|])
 // when the tables are given (the type-1 deconvolve, as k_deconvolve; kp may
 // be null: a factor 1, the 2D case), else 1.
+// b: the tile of plane p of transform t.
 template <typename T, int W, bool SCALE>
-__global__ void __launch_bounds__(256)
-k_prune_gather(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, PruneGather d,
-               const T *__restrict__ kr, const T *__restrict__ kp, const T *__restrict__ kc)
+__device__ __forceinline__ void
+prune_gather_tile(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, const PruneGather &d,
+                  const T *__restrict__ kr, const T *__restrict__ kp, const T *__restrict__ kc,
+                  int b, int p, long long t, cpx<T> (*tile)[W + 1])
 {
-    __shared__ cpx<T> tile[W][W + 1];
     constexpr int ROWS = 256 / W, PER = W / ROWS;
     const int nrt = (d.R + W - 1) / W;
-    const int r0 = (int)(blockIdx.x % nrt) * W, c0 = (int)(blockIdx.x / nrt) * W;
-    const int p = blockIdx.y;
-    const long long t = blockIdx.z;
+    const int r0 = b % nrt * W, c0 = b / nrt * W;
     const int tx = threadIdx.x % W, ty = threadIdx.x / W;
     // all PER loads of a thread in flight together, then into the tile
     {
@@ -96,23 +95,48 @@ k_prune_gather(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, PruneGat
     }
 }
 
+template <typename T, int W, bool SCALE>
+__global__ void __launch_bounds__(256)
+k_prune_gather(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, PruneGather d,
+               const T *__restrict__ kr, const T *__restrict__ kp, const T *__restrict__ kc)
+{
+    __shared__ cpx<T> tile[W][W + 1];
+    prune_gather_tile<T, W, SCALE>(in, out, d, kr, kp, kc, blockIdx.x, blockIdx.y, blockIdx.z,
+                                   tile);
+}
+
+// The gathers of all members of a plan group in one launch: workgroup b does tile
+// map[b].y of member map[b].x.  48 images of 64^2 to 512^2 took 48 launches of 4 - 5
+// us on four queues for each of the two gathers; with the zero fill, 876 -> 747 us for
+// the whole group.
+template <typename T, int W, bool SCALE>
+__global__ void __launch_bounds__(256)
+k_prune_gather_group(const PruneItem<T, PruneGather> *__restrict__ items,
+                     const int2 *__restrict__ map)
+{
+    __shared__ cpx<T> tile[W][W + 1];
+    const int2 m = map[blockIdx.x];
+    const PruneItem<T, PruneGather> &it = items[m.x];
+    const PruneGather d = it.d;
+    const int nt = prune_tiles(d, W), q = m.y / nt;
+    prune_gather_tile<T, W, SCALE>(it.in, it.out, d, it.kr, it.kp, it.kc, m.y - q * nt, q % d.P,
+                                   q / d.P, tile);
+}
+
 // out[t][p][r][c] for every c < C: s * w * in[t][c'][p][r] where c holds a
 // mode (c' as in k_prune_gather), 0 elsewhere.  With the tables given, s is
 // 1 / the kernel's Fourier series product (the type-2 amplify, as k_amplify)
 // and, for wsel 0 / 1 / 2, w = i * wsign * the frequency along r / p / c (the
 // derivative modes of execute_grad); else s = w = 1.
 template <typename T, int W, bool SCALE>
-__global__ void __launch_bounds__(256)
-k_prune_scatter(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, PruneScatter d,
-                const T *__restrict__ kr, const T *__restrict__ kp, const T *__restrict__ kc,
-                int wsel, int wsign)
+__device__ __forceinline__ void
+prune_scatter_tile(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, const PruneScatter &d,
+                   const T *__restrict__ kr, const T *__restrict__ kp, const T *__restrict__ kc,
+                   int wsel, int wsign, int b, int p, long long t, cpx<T> (*tile)[W + 1])
 {
-    __shared__ cpx<T> tile[W][W + 1];
     constexpr int ROWS = 256 / W, PER = W / ROWS;
     const int nrt = (d.R + W - 1) / W;
-    const int r0 = (int)(blockIdx.x % nrt) * W, c0 = (int)(blockIdx.x / nrt) * W;
-    const int p = blockIdx.y;
-    const long long t = blockIdx.z;
+    const int r0 = b % nrt * W, c0 = b / nrt * W;
     const int tx = threadIdx.x % W, ty = threadIdx.x / W;
     {
         const int r = r0 + tx;
@@ -167,6 +191,48 @@ k_prune_scatter(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, PruneSc
     }
 }
 
+template <typename T, int W, bool SCALE>
+__global__ void __launch_bounds__(256)
+k_prune_scatter(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, PruneScatter d,
+                const T *__restrict__ kr, const T *__restrict__ kp, const T *__restrict__ kc,
+                int wsel, int wsign)
+{
+    __shared__ cpx<T> tile[W][W + 1];
+    prune_scatter_tile<T, W, SCALE>(in, out, d, kr, kp, kc, wsel, wsign, blockIdx.x, blockIdx.y,
+                                    blockIdx.z, tile);
+}
+
+// As k_prune_gather_group.
+template <typename T, int W, bool SCALE>
+__global__ void __launch_bounds__(256)
+k_prune_scatter_group(const PruneItem<T, PruneScatter> *__restrict__ items,
+                      const int2 *__restrict__ map)
+{
+    __shared__ cpx<T> tile[W][W + 1];
+    const int2 m = map[blockIdx.x];
+    const PruneItem<T, PruneScatter> &it = items[m.x];
+    const PruneScatter d = it.d;
+    const int nt = prune_tiles(d, W), q = m.y / nt;
+    prune_scatter_tile<T, W, SCALE>(it.in, it.out, d, it.kr, it.kp, it.kc, -1, 1, m.y - q * nt,
+                                    q % d.P, q / d.P, tile);
+}
+
+// Clears kZeroChunk cells from cell kZeroChunk * map[b].y of member map[b].x on.
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_zero_group(const PruneItem<T, long long> *__restrict__ items, const int2 *__restrict__ map)
+{
+    const int2 m = map[blockIdx.x];
+    const PruneItem<T, long long> it = items[m.x];
+    const long long first = (long long)m.y * kZeroChunk;
+    cpx<T> zero;
+    zero.x = 0;
+    zero.y = 0;
+#pragma unroll
+    for (int k = 0; k < kZeroChunk; k += 256)
+        if (first + k + threadIdx.x < it.d) it.out[first + k + threadIdx.x] = zero;
+}
+
 template <typename T>
 int run_prune_gather(const cpx<T> *in, cpx<T> *out, const PruneGather &d, int ntr,
                      const T *kr, const T *kp, const T *kc, const Launch &L)
@@ -202,12 +268,45 @@ int run_prune_scatter(const cpx<T> *in, cpx<T> *out, const PruneScatter &d, int 
     return ok_or_err();
 }
 
+template <typename T> int group_tile_edge() { return prune_w<T>(); }
+
+template <typename T>
+int run_zero_group(const GroupPass &g, const Launch &L)
+{
+    k_zero_group<T><<<g.tiles, 256, 0, L.stream>>>(
+        static_cast<const PruneItem<T, long long> *>(g.items), g.map);
+    return ok_or_err();
+}
+
+template <typename T>
+int run_prune_group(int type, const GroupPass &g, bool scale, const Launch &L)
+{
+    constexpr int W = prune_w<T>();
+    if (type == 1) {
+        const auto *it = static_cast<const PruneItem<T, PruneGather> *>(g.items);
+        if (scale)
+            k_prune_gather_group<T, W, true><<<g.tiles, 256, 0, L.stream>>>(it, g.map);
+        else
+            k_prune_gather_group<T, W, false><<<g.tiles, 256, 0, L.stream>>>(it, g.map);
+    } else {
+        const auto *it = static_cast<const PruneItem<T, PruneScatter> *>(g.items);
+        if (scale)
+            k_prune_scatter_group<T, W, true><<<g.tiles, 256, 0, L.stream>>>(it, g.map);
+        else
+            k_prune_scatter_group<T, W, false><<<g.tiles, 256, 0, L.stream>>>(it, g.map);
+    }
+    return ok_or_err();
+}
+
 #define CFA_PRUNE_INST(T)                                                                   \
     template int run_prune_gather<T>(const cpx<T> *, cpx<T> *, const PruneGather &, int,    \
                                      const T *, const T *, const T *, const Launch &);      \
     template int run_prune_scatter<T>(const cpx<T> *, cpx<T> *, const PruneScatter &, int,  \
                                       const T *, const T *, const T *, int, int,            \
-                                      const Launch &);
+                                      const Launch &);                                      \
+    template int group_tile_edge<T>();                                                      \
+    template int run_zero_group<T>(const GroupPass &, const Launch &);                      \
+    template int run_prune_group<T>(int, const GroupPass &, bool, const Launch &);
 CFA_PRUNE_INST(float)
 CFA_PRUNE_INST(double)
 #undef CFA_PRUNE_INST

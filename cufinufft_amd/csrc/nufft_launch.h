@@ -283,6 +283,35 @@ struct PruneScatter {
     long long out_t = 0, op = 0, orr = 0;  // output strides (c unit)
     int R = 0, P = 0, Nc = 0, C = 0, kneg = 0, hr = 0, hp = 0;
 };
+// Tiles (edge W) of one plane of a pass.
+__host__ __device__ inline int prune_tiles(const PruneGather &d, int W)
+{
+    return ((d.R + W - 1) / W) * ((d.Nc + W - 1) / W);
+}
+__host__ __device__ inline int prune_tiles(const PruneScatter &d, int W)
+{
+    return ((d.R + W - 1) / W) * ((d.C + W - 1) / W);
+}
+// One member of a pass that a plan group runs as one launch (D: the transpose, or the
+// cells to clear), and the pass: map[b] = (member, its tile) of workgroup b.
+template <typename T, class D> struct PruneItem {
+    const cpx<T> *in;
+    cpx<T> *out;
+    D d;
+    const T *kr, *kp, *kc;
+};
+struct GroupPass {
+    void *items = nullptr;
+    int2 *map = nullptr;
+    int tiles = 0;
+};
+constexpr int kZeroChunk = 4096;  // cells a workgroup clears
+template <typename T> int group_tile_edge();
+template <typename T> int run_zero_group(const GroupPass &g, const Launch &L);
+// type 1: gathers, type 2: scatters; scale: with the Fourier-series tables.
+template <typename T>
+int run_prune_group(int type, const GroupPass &g, bool scale, const Launch &L);
+
 // Cell of mode index q (frequency q - kneg) on an axis of C cells, and the
 // mode index of cell c (-1 where the cell holds no mode); Nc modes, the kneg
 // negative frequencies at the top of the axis.

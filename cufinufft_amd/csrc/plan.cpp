@@ -1420,10 +1420,19 @@ struct Group {
     static constexpr int kBranches = 4;
     hipStream_t br[kBranches] = {};
     hipEvent_t ev_fork = nullptr, ev_join[kBranches] = {};
+    // Where every member's FFT is pruned (2D, 3D) the zero fill and the transposes
+    // between the FFT passes run as one launch over all members each; only the
+    // FFTs stay per member.
+    bool staged = false;
+    GroupPass zero, pass[3];
 
     ~Group()
     {
         DeviceGuard dg(dev);
+        for (GroupPass *g : {&zero, &pass[0], &pass[1], &pass[2]}) {
+            if (g->items) hipFree(g->items);
+            if (g->map) hipFree(g->map);
+        }
         if (gexec) hipGraphExecDestroy(gexec);
         if (graph) hipGraphDestroy(graph);
         if (ev_in) hipEventDestroy(ev_in);
@@ -1496,7 +1505,114 @@ struct Group {
             return kErrHip;
         if (hipMemcpy(items, h.data(), h.size(), hipMemcpyHostToDevice) != hipSuccess)
             return kErrHip;
-        return 0;
+        staged = dim >= 2;
+        for (const auto *p : plans) staged = staged && p->pruned;
+        return staged ? make_passes() : 0;
+    }
+
+    // Uploads a pass: its items and, per item, the number of workgroups.
+    template <class Item>
+    int upload(GroupPass &g, const std::vector<Item> &it, const std::vector<long long> &tiles)
+    {
+        std::vector<int2> map;
+        for (size_t i = 0; i < it.size(); ++i)
+            for (long long k = 0; k < tiles[i]; ++k) map.push_back(make_int2((int)i, (int)k));
+        g.tiles = (int)map.size();
+        return hipMalloc(&g.items, sizeof(Item) * it.size()) == hipSuccess &&
+                       hipMalloc((void **)&g.map, sizeof(int2) * map.size()) == hipSuccess &&
+                       hipMemcpy(g.items, it.data(), sizeof(Item) * it.size(),
+                                 hipMemcpyHostToDevice) == hipSuccess &&
+                       hipMemcpy(g.map, map.data(), sizeof(int2) * map.size(),
+                                 hipMemcpyHostToDevice) == hipSuccess
+                   ? 0
+                   : kErrHip;
+    }
+    // Transpose k of every member; D: PruneGather (type 1) or PruneScatter (type 2).
+    template <class D, class F>
+    int make_pass(int k, F &&describe)
+    {
+        const int W = group_tile_edge<T>();
+        std::vector<PruneItem<T, D>> it;
+        std::vector<long long> tiles;
+        for (size_t i = 0; i < plans.size(); ++i) {
+            it.push_back(describe(*plans[i], fk[i]));
+            tiles.push_back((long long)prune_tiles(it[i].d, W) * it[i].d.P * plans[i]->ntransf);
+        }
+        return upload(pass[k], it, tiles);
+    }
+    int make_passes()
+    {
+        using P = Plan<T>;
+        using G = PruneItem<T, PruneGather>;
+        using S = PruneItem<T, PruneScatter>;
+        // the map of the largest pass: 8 bytes per tile or 4096 cells, at most 64 MiB
+        long long work = 0;
+        for (const P *p : plans) {
+            const int W = group_tile_edge<T>();
+            const long long lines = (long long)p->nf[2] * p->ntransf;
+            work += (p->nf[0] / W + 1ll) * (p->nf[1] / W + 1ll) * lines;
+            if (dim == 3)
+                work += (p->nf[0] / W + 1ll) * (p->nf[2] / W + 1ll) * p->nf[1] * p->ntransf +
+                        (p->nf[1] / W + 1ll) * (p->nf[2] / W + 1ll) * p->nf[0] * p->ntransf;
+        }
+        if (work > 1 << 23) {
+            staged = false;
+            return 0;
+        }
+        int e = 0;
+        if (type == 1) {
+            std::vector<PruneItem<T, long long>> it;
+            std::vector<long long> tiles;
+            for (P *p : plans) {
+                it.push_back({nullptr, p->fw, p->nftot * p->ntransf, nullptr, nullptr, nullptr});
+                tiles.push_back((it.back().d + kZeroChunk - 1) / kZeroChunk);
+            }
+            e = upload(zero, it, tiles);
+            if (!e && dim == 2) {
+                e = make_pass<PruneGather>(0, [](P &p, cpx<T> *) {
+                    return G{p.fw, p.fwh, prune2_fw_to_b1(p.ms, p.nf), nullptr, nullptr, nullptr};
+                });
+                if (!e)
+                    e = make_pass<PruneGather>(1, [](P &p, cpx<T> *f) {
+                        return G{p.fwh,      f,       prune2_b1_to_fk(p.ms, p.nf),
+                                 p.fwker[0], nullptr, p.fwker[1]};
+                    });
+            } else if (!e) {
+                e = make_pass<PruneGather>(0, [](P &p, cpx<T> *) {
+                    return G{p.fw, p.fwh, prune_fw_to_b1(p.ms, p.nf), nullptr, nullptr, nullptr};
+                });
+                if (!e)
+                    e = make_pass<PruneGather>(1, [](P &p, cpx<T> *) {
+                        return G{p.fwh, p.fw, prune_b1_to_b2(p.ms, p.nf), nullptr, nullptr, nullptr};
+                    });
+                if (!e)
+                    e = make_pass<PruneGather>(2, [](P &p, cpx<T> *f) {
+                        return G{p.fw,       f,          prune_b2_to_fk(p.ms, p.nf),
+                                 p.fwker[0], p.fwker[1], p.fwker[2]};
+                    });
+            }
+        } else if (dim == 2) {
+            e = make_pass<PruneScatter>(0, [](P &p, cpx<T> *f) {
+                return S{f, p.fwh, prune2_fk_to_b1(p.ms, p.nf), p.fwker[0], nullptr, p.fwker[1]};
+            });
+            if (!e)
+                e = make_pass<PruneScatter>(1, [](P &p, cpx<T> *) {
+                    return S{p.fwh, p.fw, prune2_b1_to_fw(p.ms, p.nf), nullptr, nullptr, nullptr};
+                });
+        } else {
+            e = make_pass<PruneScatter>(0, [](P &p, cpx<T> *f) {
+                return S{f, p.fw, prune_fk_to_b2(p.ms, p.nf), p.fwker[0], p.fwker[1], p.fwker[2]};
+            });
+            if (!e)
+                e = make_pass<PruneScatter>(1, [](P &p, cpx<T> *) {
+                    return S{p.fw, p.fwh, prune_b2_to_b1(p.ms, p.nf), nullptr, nullptr, nullptr};
+                });
+            if (!e)
+                e = make_pass<PruneScatter>(2, [](P &p, cpx<T> *) {
+                    return S{p.fwh, p.fw, prune_b1_to_fw(p.ms, p.nf), nullptr, nullptr, nullptr};
+                });
+        }
+        return e;
     }
 
     // The launch sequence, on the group stream.
@@ -1539,7 +1655,29 @@ struct Group {
                     return kErrHip;
             return err;
         };
-        if (type == 1) {
+        // the 1D FFTs of axis a of every member (y passes run in fwh)
+        auto ffts = [&](int a) {
+            return branches([&](int i, const Launch &) {
+                Plan<T> &p = *plans[i];
+                typename Plan<T>::Fft1d *f = nullptr;
+                const int err = p.fft1d(f, p.ntransf);
+                return err ? err : p.exec1d(f->h[a], a == 1 ? p.fwh : p.fw);
+            });
+        };
+        if (staged && type == 1) {
+            e = run_zero_group<T>(zero, L);
+            if (!e) e = spread_or_interp();
+            for (int a = 0; a < dim && !e; ++a) {
+                e = ffts(a);
+                if (!e) e = run_prune_group<T>(1, pass[a], a == dim - 1, L);
+            }
+        } else if (staged) {
+            for (int a = dim - 1; a >= 0 && !e; --a) {
+                e = run_prune_group<T>(2, pass[dim - 1 - a], a == dim - 1, L);
+                if (!e) e = ffts(a);
+            }
+            if (!e) e = spread_or_interp();
+        } else if (type == 1) {
             e = branches([&](int i, const Launch &Lb) {
                 return run_zero<T>(plans[i]->fw, plans[i]->nftot * plans[i]->ntransf, Lb);
             });
