@@ -41,6 +41,14 @@ struct WinPts {
     const int2 *range;    // first point of each range (ranges + 1) and its window
     long long stride;
 };
+// A member's transform in a plan group's window spread.
+template <typename T, class Geom = BinGeom> struct WinItem {
+    WinPts wp;
+    const cpx<T> *c;
+    cpx<T> *fw;
+    Geom g;
+    WinGeom wg;
+};
 constexpr int kWinPack = 64;      // bytes of a point's packed strengths
 constexpr int kWinKeyWeight = 8;  // a window's own time in a range, in points
 // Half of a 3D interp window's y and z extent: windows of 8 cells up to ns 8,
@@ -173,6 +181,13 @@ constexpr bool win_interp_width(int, int ns, size_t elem)
 // ones), and the window order of the points after run_bin_sort.
 WinGeom win_choose(int type, int dim, int ns, int elem, const BinGeom &g, int M, int ntr, int ncu);
 int run_win_clear(const SortBufs &sb, long long keys, const Launch &L);  // wcount = 0
+// Windows of a 2D type-1 plan group's member and its work (in points: a window's
+// flush takes about as long as 24; with ranges by points alone a sparse member's few
+// waves ran on alone, 48 images took 1139 us instead of 516).
+WinGeom win_member(int ns, int elem, const BinGeom &g, int M, double &work);
+template <typename T>
+int run_win_group(int ns, const void *items, const int2 *map, int waves, const KerParams<T> &kp,
+                  const Launch &L);
 template <typename T>
 int run_win_sort(int dim, int M, const SortBufs &sb, const Launch &L);
 template <typename T, int DIM>

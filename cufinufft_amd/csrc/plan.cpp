@@ -715,6 +715,7 @@ struct Plan {
                        size_t scr_bytes);
     int setpts_blocks();
     WinGeom choose_win(int M_) const;
+    long long npts_set = 0;  // setpts calls so far
     long long cap_wkeys = -1, cap_wM = -1, cap_wranges = -1;  // of the window order
     int alloc_win();
     void free_win()
@@ -1111,6 +1112,7 @@ int Plan<T>::setpts(int M_, const T *x, const T *y, const T *z)
     kx = x;
     ky = dim > 1 ? y : nullptr;
     kz = dim > 2 ? z : nullptr;
+    ++npts_set;
     if (M > cap_M && method != 4) {
         dfree(sb.skey);
         dfree(sb.skey_out);
@@ -1228,6 +1230,7 @@ int Plan<T>::setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned
     kx = x;
     ky = dim > 1 ? y : nullptr;
     kz = dim > 2 ? z : nullptr;
+    ++npts_set;
     sub_bound = sub_need;
     sb.win = win;
     int e;
@@ -1425,11 +1428,17 @@ struct Group {
     // FFTs stay per member.
     bool staged = false;
     GroupPass zero, pass[3];
+    // 2D type 1: the members' points in window order (one block of memory), for as
+    // long as no member's points are set again
+    GroupPass win;
+    void *win_mem = nullptr;
+    std::vector<long long> win_pts;  // the members' setpts counts at make time
 
     ~Group()
     {
         DeviceGuard dg(dev);
-        for (GroupPass *g : {&zero, &pass[0], &pass[1], &pass[2]}) {
+        if (win_mem) hipFree(win_mem);
+        for (GroupPass *g : {&zero, &pass[0], &pass[1], &pass[2], &win}) {
             if (g->items) hipFree(g->items);
             if (g->map) hipFree(g->map);
         }
@@ -1507,7 +1516,96 @@ struct Group {
             return kErrHip;
         staged = dim >= 2;
         for (const auto *p : plans) staged = staged && p->pruned;
-        return staged ? make_passes() : 0;
+        const int e = staged ? make_passes() : 0;
+        return e ? e : make_win();
+    }
+
+    // Orders every member's points by window (2D type 1); without the memory, or
+    // where a member's windows would wrap twice, the subproblem kernel spreads.
+    int make_win()
+    {
+        if (type != 1 || dim != 2) return 0;
+        double total = 0;
+        std::vector<double> work(plans.size(), 0);
+        std::vector<SortBufs> sb;
+        size_t bytes = 0;
+        std::vector<size_t> at;
+        for (size_t i = 0; i < plans.size(); ++i) {
+            const Plan<T> &p = *plans[i];
+            SortBufs s = p.sb;
+            s.win = win_member(ns, sizeof(T), p.geom, p.M, work[i]);
+            if (p.M > 0 && s.win.ranges == 0) return 0;
+            total += work[i] * p.ntransf;
+            sb.push_back(s);
+        }
+        // two rounds of the waves resident on the device
+        const double per = std::max(256.0, total / (2.0 * L.ncu * (sizeof(T) == 4 ? 16 : 8)));
+        for (size_t i = 0; i < sb.size(); ++i)
+            if (sb[i].win.ranges)
+                sb[i].win.ranges = (int)std::min((double)plans[i]->M, std::ceil(work[i] / per));
+        auto take = [&](size_t n) {
+            at.push_back(bytes);
+            bytes += (n + 255) / 256 * 256;
+        };
+        for (const SortBufs &s : sb) {
+            const size_t k = s.win.nkeys, m = s.pos_stride;
+            take(4 * k);
+            take(4 * (k + 1));
+            take(4 * (k + 1));
+            take(sizeof(int2) * (k / kScanChunk + 3));
+            take(sizeof(int2) * (s.win.ranges + 1));
+            take(sizeof(T) * dim * m);
+            take(4 * m);
+            take(4 * m);
+        }
+        if (hipMalloc(&win_mem, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            win_mem = nullptr;
+            return 0;
+        }
+        std::vector<WinItem<T>> it;
+        std::vector<long long> waves;
+        for (size_t i = 0; i < sb.size(); ++i) {
+            SortBufs &s = sb[i];
+            auto ptr = [&](int k) { return static_cast<char *>(win_mem) + at[8 * i + k]; };
+            s.wcount = reinterpret_cast<int *>(ptr(0));
+            s.wstart = reinterpret_cast<int *>(ptr(1));
+            s.wused = reinterpret_cast<int *>(ptr(2));
+            s.wpart = ptr(3);
+            s.wrange = reinterpret_cast<int2 *>(ptr(4));
+            s.wx = ptr(5);
+            s.wsh = reinterpret_cast<unsigned *>(ptr(6));
+            s.widx = reinterpret_cast<int *>(ptr(7));
+            Plan<T> &p = *plans[i];
+            win_pts.push_back(p.npts_set);
+            if (p.M == 0) continue;
+            // after the member's own setpts, on its stream
+            if (run_win_clear(s, s.win.nkeys, p.L) || run_win_sort<T>(dim, p.M, s, p.L) ||
+                hipStreamSynchronize(p.L.stream) != hipSuccess)
+                return kErrHip;
+            for (int t = 0; t < p.ntransf; ++t) {
+                it.push_back({WinPts{s.wx, s.wsh, s.widx, s.wstart, s.wrange, s.pos_stride},
+                              c[i] + (long long)t * p.M, p.fw + (long long)t * p.nftot, p.geom,
+                              s.win});
+                waves.push_back(s.win.ranges);
+            }
+        }
+        return it.empty() ? 0 : upload(win, it, waves);
+    }
+    // Whether the window order still is that of the members' points; if not, it is
+    // dropped, and a graph that holds it.
+    int check_win()
+    {
+        bool ok = true;
+        for (size_t i = 0; i < win_pts.size(); ++i) ok = ok && win_pts[i] == plans[i]->npts_set;
+        if (ok || !win.tiles) return 0;
+        win.tiles = 0;
+        if (hipStreamSynchronize(stream) != hipSuccess) return kErrHip;
+        if (gexec && hipGraphExecDestroy(gexec) != hipSuccess) return kErrHip;
+        gexec = nullptr;
+        if (graph && hipGraphDestroy(graph) != hipSuccess) return kErrHip;
+        graph = nullptr;
+        return 0;
     }
 
     // Uploads a pass: its items and, per item, the number of workgroups.
@@ -1631,6 +1729,7 @@ struct Group {
             plans[i]->L.stream = stream;  // the members' FFTs run on the group stream
         }
         auto spread_or_interp = [&]() {
+            if (win.tiles) return run_win_group<T>(ns, win.items, win.map, win.tiles, kp, L);
             if (dim == 1)
                 return group_dim<T, 1>(type, ns, items, n, off, kp, bs, maxsub, jobs_bound, L);
             if (dim == 2)
@@ -1708,6 +1807,7 @@ struct Group {
     {
         ApiRange ar("cufinufft_group_execute");
         DeviceGuard dg(dev);
+        if (check_win()) return kErrHip;
         if (hipEventRecord(ev_in, user) != hipSuccess ||
             hipStreamWaitEvent(stream, ev_in, 0) != hipSuccess)
             return kErrHip;

@@ -448,36 +448,37 @@ k_win_pack(int M, int nt, const cpx<T> *__restrict__ c, cpx<T> *__restrict__ out
     for (int t = 0; t < NT; ++t) out[(long long)NT * i + t] = v[t];
 }
 
-// Point id's strength of transform t is c[t ct + id ci].
+// LDS of a wave.
 template <typename T, int DIM, int NS, int NT>
-__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
-k_win_spread(WinPts wp, const cpx<T> *__restrict__ c, long long ct, int ci, cpx<T> *__restrict__ fw,
-             BinGeom g, WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
+struct WinSpreadLds {
+    static constexpr int B = WinSpread<T, DIM, NS, NT>::kBlock;
+    alignas(16) cpx<T> cs[B * NT];
+    cpx<T> sc[256];
+    unsigned sh[B];
+    T rows[B * WinRow<T, DIM, NS>::pitch];
+};
+
+// One wave spreads range rng of a window order: nt <= NT transforms; point id's
+// strength of transform t is c[t ct + id ci].
+template <typename T, int DIM, int NS, int NT>
+__device__ __forceinline__ void
+win_spread_range(int rng, const WinPts &wp, const cpx<T> *__restrict__ c, long long ct, int ci,
+                 T *__restrict__ ft, const BinGeom &g, const WinGeom &wg, const KerParams<T> &kp,
+                 int nt, long long nftot, WinSpreadLds<T, DIM, NS, NT> &lds)
 {
     constexpr int F = (NS + 1) / 2 + 1, S = 17 - NS;
     using Acc = WinSpread<T, DIM, NS, NT>;
     using Row = WinRow<T, DIM, NS>;
     constexpr int B = Acc::kBlock;
-    __shared__ T srow[4 * B * Row::pitch];
-    __shared__ unsigned ssh[4 * B];
-    __shared__ alignas(16) cpx<T> scs[4 * B * NT];
-    __shared__ cpx<T> ssc[1024];
     const int lane = threadIdx.x & 63, h = lane >> 5, pl = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    T *rows = srow + wave * B * Row::pitch;
-    unsigned *sh = ssh + wave * B;
-    cpx<T> *cs = scs + wave * B * NT, *sc = ssc + wave * 256;
+    T *rows = lds.rows;
+    unsigned *sh = lds.sh;
+    cpx<T> *cs = lds.cs, *sc = lds.sc;
     const T *x1 = static_cast<const T *>(wp.x);
-    const JobRange jr = xcd_jobs(gridDim.x);  // one range per wave, contiguous per XCD
-    const int rng = (int)jr.begin * 4 + wave;
-    if (rng >= wg.ranges) return;
     const int2 r0 = wp.range[rng];
     int p = r0.x;
     const int pe = wp.range[rng + 1].x;
     if (p >= pe) return;
-    const int t0 = blockIdx.y * NT, nt = min(NT, ntr - t0);
-    c += t0 * ct;
-    T *ft = reinterpret_cast<T *>(fw + (long long)t0 * nftot);
     const double back = exp((double)DIM * (double)kp.beta);
     Acc acc;
     acc.clear();
@@ -574,6 +575,43 @@ k_win_spread(WinPts wp, const cpx<T> *__restrict__ c, long long ct, int ci, cpx<
             p = e;
         }
     }
+}
+
+template <typename T, int DIM, int NS, int NT>
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
+k_win_spread(WinPts wp, const cpx<T> *__restrict__ c, long long ct, int ci, cpx<T> *__restrict__ fw,
+             BinGeom g, WinGeom wg, KerParams<T> kp, int ntr, long long nftot)
+{
+    __shared__ WinSpreadLds<T, DIM, NS, NT> lds[4];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const JobRange jr = xcd_jobs(gridDim.x);  // one range per wave, contiguous per XCD
+    const int rng = (int)jr.begin * 4 + wave;
+    if (rng >= wg.ranges) return;
+    const int t0 = blockIdx.y * NT;
+    win_spread_range<T, DIM, NS, NT>(rng, wp, c + t0 * ct, ct, ci,
+                                     reinterpret_cast<T *>(fw + (long long)t0 * nftot), g, wg, kp,
+                                     min(NT, ntr - t0), nftot, lds[wave]);
+}
+
+// The ranges of all members of a plan group: wave w takes range map[w].y of item
+// map[w].x (a member's transform).
+template <typename T, int NS>
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2)
+k_win_spread_group(const WinItem<T> *__restrict__ items, const int2 *__restrict__ map, int waves,
+                   KerParams<T> kp)
+{
+    __shared__ WinSpreadLds<T, 2, NS, 1> lds[4];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // neighbouring windows on one XCD
+    const int w = (int)xcd_jobs(gridDim.x).begin * 4 + wave;
+    if (w >= waves) return;
+    const int2 m = map[w];
+    const WinItem<T> &it = items[m.x];
+    const WinPts wp = it.wp;
+    const BinGeom g = it.g;
+    const WinGeom wg = it.wg;
+    win_spread_range<T, 2, NS, 1>(m.y, wp, it.c, 0, 1, reinterpret_cast<T *>(it.fw), g, wg, kp, 1,
+                                  0, lds[wave]);
 }
 
 // ---------------------------------------------------------------------------

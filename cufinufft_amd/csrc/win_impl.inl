@@ -14,9 +14,9 @@ inline WinPts win_pts(const SortBufs &sb)
     return WinPts{sb.wx, sb.wsh, sb.widx, sb.wstart, sb.wrange, sb.pos_stride};
 }
 // Workgroups of 4 waves, a range each; whole XCD groups.
-inline int win_grid(const WinGeom &w)
+inline int win_grid(int ranges)
 {
-    const int grid = (w.ranges + 3) / 4;
+    const int grid = (ranges + 3) / 4;
     return grid >= kNumXcd ? (grid + kNumXcd - 1) / kNumXcd * kNumXcd : grid;
 }
 
@@ -27,7 +27,7 @@ int win_spread_ns(int M, const SortBufs &sb, const cpx<T> *c, cpx<T> *fw, const 
     if constexpr (!win_spread_width(DIM, NS, sizeof(T))) {
         return 1;
     } else {
-        const int grid = win_grid(sb.win);
+        const int grid = win_grid(sb.win.ranges);
         constexpr int P = DIM == 2 ? kWinPack / (int)sizeof(cpx<T>) : 1;
         if (DIM == 2 && ntr >= 4 && sb.wc) {
             cpx<T> *pk = static_cast<cpx<T> *>(sb.wc);
@@ -57,7 +57,7 @@ int win_interp_ns(int M, const SortBufs &sb, cpx<T> *c, const cpx<T> *fw, const 
     if constexpr (!win_interp_width(DIM, NS, sizeof(T))) {
         return 1;
     } else {
-        k_win_interp<T, DIM, NS><<<win_grid(sb.win), 256, 0, L.stream>>>(
+        k_win_interp<T, DIM, NS><<<win_grid(sb.win.ranges), 256, 0, L.stream>>>(
             M, win_pts(sb), c, fw, g, sb.win, kp, ntr, nftot);
         return hipGetLastError() == hipSuccess ? 0 : kErrHip;
     }
@@ -82,6 +82,26 @@ int win_spread_dim(int ns, int M, const SortBufs &sb, const cpx<T> *c, cpx<T> *f
 #undef CFA_CASE
     }
     return 1;
+}
+
+template <typename T>
+int win_group_ns(int ns, const void *items, const int2 *map, int waves, const KerParams<T> &kp,
+                 const Launch &L)
+{
+    const WinItem<T> *it = static_cast<const WinItem<T> *>(items);
+    switch (ns) {
+#define CFA_CASE(N)                                                                          \
+    case N:                                                                                  \
+        if constexpr (win_spread_width(2, N, sizeof(T)))                                     \
+            k_win_spread_group<T, N><<<win_grid(waves), 256, 0, L.stream>>>(it, map, waves,  \
+                                                                            kp);             \
+        break;
+        CFA_NS_CASES(CFA_CASE)
+#undef CFA_CASE
+    default:
+        return 1;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : kErrHip;
 }
 
 template <typename T, int DIM>

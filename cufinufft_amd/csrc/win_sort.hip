@@ -153,6 +153,20 @@ WinGeom win_choose(int type, int dim, int ns, int elem, const BinGeom &g, int M,
     return w;
 }
 
+// A 2D type-1 plan group spreads by window wherever the kernels are built (the order
+// is made with the group): 48 images of 64^2 to 512^2 with up to 1e6 points each,
+// FP32, ns 7, took 788 us by the subproblem kernel and 516 us by window (whole
+// group), ns 5: 706 and 482; with up to 1e4 points, 2 per window, 527 and 319; 5
+// images, 114 and 112; 30 FP64 images, ns 10, up to 3e5 points, 528 and 375.
+WinGeom win_member(int ns, int elem, const BinGeom &g, int M, double &work)
+{
+    WinGeom w, none;
+    if (M <= 0 || !win_spread_width(2, ns, elem) || !win_windows(1, 2, ns, g.nf, w)) return none;
+    w.ranges = 1;
+    work = M + 24.0 * std::min(M, w.nkeys);
+    return w;
+}
+
 int run_win_clear(const SortBufs &sb, long long keys, const Launch &L)
 {
     const long long b = (keys + 255) / 256;

@@ -45,3 +45,36 @@ def test_group_passes(torch_dev, dim, typ, dtype, tol, graph):
         torch.cuda.synchronize()
         for o, w in zip(outs, want):
             assert (o - w).abs().max() <= 50 * np.finfo(dtype).eps * w.abs().max()
+
+
+@pytest.mark.parametrize("dtype,tol,bar", [(np.float32, 1e-6, 2e-6), (np.float64, 1e-9, 1e-12)])
+@pytest.mark.parametrize("graph", [False, True])
+def test_group_window_spread(torch_dev, dtype, tol, bar, graph):
+    """Type-1 groups whose members' points fill the windows, against each member's own
+    execute (relative L2; weights and sums of either path agree to rounding), also
+    after a member's points were set again."""
+    import torch
+    from cufinufft_amd import cufinufft
+    from cufinufft_amd.cufinufft import cufinufft_group
+    plans, cs, fks, sizes = [], [], [], [(33, 40), (64, 51), (97, 16), (20, 130)]
+    for k, nm in enumerate(sizes):
+        m, ntr = 60001 + 1777 * k, 1 + k % 3
+        plan = cufinufft(1, nm, n_trans=ntr, eps=tol, dtype=dtype, gpu_method=2, maxbatchsize=ntr)
+        pts = (G.uniform_pts if k % 2 else G.clustered_pts)(m, 2, dtype, 3 + k)
+        plan.set_pts(*[G.to_dev(p, torch_dev) for p in pts])
+        plans.append(plan)
+        cs.append(G.to_dev(G.strengths(m, dtype, k, ntr), torch_dev))
+        fks.append(torch.empty((ntr,) + nm, dtype=cs[-1].dtype, device=torch_dev))
+    group = cufinufft_group(plans, cs, fks)
+    for again in range(3):
+        if again == 2:  # other points of a member
+            m = cs[1].numel() // plans[1].n_trans
+            plans[1].set_pts(*[G.to_dev(p, torch_dev) for p in G.uniform_pts(m, 2, dtype, 77)])
+        for o in fks:
+            o.fill_(7)
+        group.execute(use_graph=graph)
+        torch.cuda.synchronize()
+        for p, c, f in zip(plans, cs, fks):
+            want = torch.empty_like(f)
+            p.execute(c, want)
+            assert (f - want).norm() < bar * want.norm()
