@@ -103,28 +103,45 @@ k_win_ranges(int M, int nkeys, int ranges, int *__restrict__ start, const int *_
 }
 
 // Where the window kernels beat the per-point ones, the window order's own time
-// in setpts (30 us, and 15-25 ns per 1000 points) included.  Measured on uniform
-// points, per-point -> window kernel:
-//  3D spread: 0.79 -> 0.29 ms (FP32, ns 6, M = 1e5 on 256^3), 2.3 -> 1.0 ms (1e7),
-//   4.0 -> 0.57 ms (ns 7, 1e6), 14.4 -> 2.8 ms (FP64, ns 10, 1e7); under ~5e4
-//   points (2e4 where the per-point kernel holds 64-bit cells) a window holds so
-//   few points that its flush costs more than their taps, and at ns 4, 5 dense
-//   grids have too few taps per point (0.62 -> 0.68 ms, ns 4, 11 points per cell).
-//  3D interp: a window's cells are read once whatever its points, so it takes
-//   some points per window: 3.1 -> 1.3 ms (FP32, ns 6, 1e7, 59 per window), 0.50
-//   -> 0.58 ms (1e6, 6 per window); FP64 3.0 -> 2.8 ms (ns 10, 4 per window).
-//  2D: few taps, so the order's time decides: 0.65 -> 0.34 ms (FP32, ns 7, 1e7,
-//   order 0.15 ms), 0.078 -> 0.046 ms (1e6, order 0.04 ms); a batch shares it.
+// (25 - 35 us for small sets, 15 - 25 ns per 1000 points) in every call included.
+// Measured per-point -> window, setpts and execute, uniform points:
+//  3D type 1, 48^3 modes: FP32 ns 5, 4e4 points 180 -> 202 us, 2e5 211 -> 169; ns 6,
+//   4e4 199 -> 177, 1e4 170 -> 247; ns 7, 1e4 342 -> 277; FP64 ns 7, 1e4 322 -> 315,
+//   ns 10 608 -> 471.  128^3: FP32 ns 6, 3e5 1409 -> 554; FP64 ns 10, 2e6 8520 -> 2128.
+//   ns 4: dense grids have too few taps per point (spread alone 0.62 -> 0.68 ms).
+//  3D type 2 reads a window's cells once whatever its points: FP32, 48^3, 2e5 points,
+//   ns 5 172 -> 168, ns 7 222 -> 199, ns 6, 4e4 156 -> 206; 128^3, 3e5, ns 6 (1.7
+//   points per window) 512 -> 504.  FP64 ns 7, 128^3, 3e5 (0.7) 929 -> 1082, 2e6 (4.7)
+//   2903 -> 1430; ns 10, 4e4 (0.14) 1007 -> 923, 48^3, 4e4 369 -> 369; ns 13, 48^3, 4e4
+//   731 -> 700, 1e4 712 -> 834, 128^3, 3e5 (0.27) 3863 -> 2718.
+//  2D type 1: FP32 ns 7, 640^2 modes, 1e6 183 -> 187, 4e6 404 -> 377, ns 6, 4e6 352 ->
+//   365; FP64 ns 7, 1e6 240 -> 235, 4e6 561 -> 533; ns 10, 256^2, 3e5 108 -> 97, 640^2,
+//   2e5 (5.9 per window) 204 -> 203; ns 13, 640^2, 2e5 (1.9) 226 -> 234, 1e6 (9.7) 345
+//   -> 298, 256^2, 1e5 80 -> 98.  32 FP32 transforms, ns 7, 2e6: 3.7 -> 1.5 ms; 4
+//   transforms of 2e5: 122 -> 138 us.
+//  2D type 2: FP32 ns 7, 640^2, 1e6 182 -> 187, 4e6 445 -> 409, ns 6, 4e6 383 -> 400;
+//   4 transforms, 320^2, 2e5, ns 5 118 -> 111, ns 7 160 -> 116; FP64 ns 7, 1e6 222 ->
+//   246, 4e6 657 -> 557; ns 10, 256^2, 1e5 78 -> 84, 3e5 116 -> 110, 640^2, 2e5 (5.9)
+//   208 -> 189; ns 13, 640^2, 2e5 (1.9) 242 -> 246, 1e6 436 -> 315.
 static bool win_pays(int type, int dim, int ns, int elem, int M, int ntr, double per_window)
 {
-    const bool wide = elem == 8 || ns >= 7;
-    if (dim == 3 && type == 1) return M >= (wide ? 20000 : 60000) && (ns >= 6 || elem == 8);
-    if (dim == 3)
-        return M >= 200000 && per_window >= (elem == 8 ? 4 : 8) && (ns >= 6 || elem == 8);
+    const bool dbl = elem == 8;
+    if (dim == 3 && type == 1) {
+        if (ns >= 7) return M >= 10000;
+        if (dbl) return M >= 20000;
+        return ns == 6 ? M >= 40000 : ns == 5 && M >= 150000;
+    }
+    if (dim == 3) {
+        if (dbl && ns >= 9) return M >= 50000 && per_window >= 0.1;
+        if (dbl) return M >= 200000 && per_window >= 4;
+        return ns >= 5 && M >= 200000 && per_window >= 1.5;
+    }
     const double taps = (double)M * ntr * ns * ns;
-    if (type == 1)
-        return per_window >= 50 && taps >= (elem == 8 ? 1e8 : 2e8) && (ns >= 7 || ntr >= 4);
-    return per_window >= 10 && taps >= (elem == 8 && ns >= 8 ? 1e8 : 4e8) && ns >= 6;
+    if (dbl && ns >= 9) return per_window >= 5 && taps >= (type == 1 ? 3e7 : 2e7);
+    if (type == 1) return per_window >= 50 && taps >= 1.5e8 && (ns >= 7 || ntr >= 4);
+    if (per_window < 10) return false;
+    if (ntr >= 4 && ns >= 5) return taps >= 2e7;
+    return ns >= 7 ? taps >= 1.5e8 : ns == 6 && taps >= 4e8;
 }
 
 WinGeom win_choose(int type, int dim, int ns, int elem, const BinGeom &g, int M, int ntr, int ncu)
