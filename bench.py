@@ -225,6 +225,16 @@ def algorithmic_bytes(w, nf, kind):
     return T * M * 2 * s + M * d * s + 4 * M + T * nftot * 2 * s
 
 
+def uses_windows(w, info):
+    """Whether the plan's points are far inside the library's rule for the
+    window kernels (large 3D sets, large 2D batches; built widths; not the
+    block method, and not the atomic method of type 1)."""
+    wide = 9 if w["dtype"] == "float32" else 13
+    return (w["dim"] >= 2 and info["method"] != 4 and not (w["type"] == 1 and info["method"] == 1)
+            and 6 <= info["ns"] <= wide and w["M"] >= 1_000_000
+            and (w["dim"] == 3 or w["ntransf"] >= 4))
+
+
 def uses_tile_slots(w, info):
     """Whether a type-1 SM plan stores single-subproblem tiles for the gather
     pass (the library's rule: every axis with >= 3 bins, a halo of
@@ -614,7 +624,10 @@ def measure(w, wname, dev, dpts, din, sel, ref, a, accuracy_first=False):
     nbytes = algorithmic_bytes(w, best["info"]["nf"], "interp" if w["type"] == 2 else "spread")
     kname = ("k_interp_" if w["type"] == 2 else "k_spread_") + \
         {1: "gm", 2: "sm", 4: "blk"}[best["info"]["method"]]
-    slots = isinstance(best_opts, dict) and best_opts.get("tile_slots", False)
+    window = uses_windows(w, best["info"])
+    if window:
+        kname = "k_win_interp" if w["type"] == 2 else "k_win_spread"
+    slots = not window and isinstance(best_opts, dict) and best_opts.get("tile_slots", False)
     kstage = kname + (" + k_tile_gather" if slots and uses_tile_slots(w, best["info"]) else "")
     # template arguments <T, [Acc,] DIM, NS[, threads]>: match by name, type and NS
     ktmpl = (kname, "float" if dt == np.float32 else "double", w["dim"], best["info"]["ns"])
