@@ -1069,13 +1069,13 @@ WinGeom Plan<T>::choose_win(int M_) const
     return win_choose(type, dim, sp.ns, sizeof(T), geom, M_, ntransf, L.ncu);
 }
 
-// Arrays of the window order for sb.win (grown on demand; x as the positions,
-// cap_M points per axis).
+// Arrays of the window order for sb.win (grown on demand; they hold pos_stride
+// points per axis, as the positions do).
 template <typename T>
 int Plan<T>::alloc_win()
 {
     const long long keys = sb.win.nkeys;
-    if (keys <= cap_wkeys && M <= cap_wM && sb.win.ranges <= cap_wranges) return 0;
+    if (keys <= cap_wkeys && sb.pos_stride == cap_wM && sb.win.ranges <= cap_wranges) return 0;
     free_win();
     const long long parts = (keys + kScanChunk - 1) / kScanChunk;
     if (dmalloc(&sb.wcount, (size_t)keys) || dmalloc(&sb.wstart, (size_t)keys + 1) ||
@@ -1203,7 +1203,8 @@ int Plan<T>::setpts_noalloc(int M_, const T *x, const T *y, const T *z, unsigned
     if (need_sub && sub_need > cap_sub) return kErrNoAlloc;
     // the window order needs its arrays too: without them the per-point kernels run
     WinGeom win = choose_win(M_);
-    if (win.nkeys > cap_wkeys || M_ > cap_wM || win.ranges > cap_wranges) win = WinGeom();
+    if (win.nkeys > cap_wkeys || sb.pos_stride != cap_wM || win.ranges > cap_wranges)
+        win = WinGeom();
     SortBufs s2 = sb;
     if (!(method == 1 && !opts.gpu_sort) && M_ > 0) {
         const long long nkeys =
